@@ -345,7 +345,7 @@ struct scratch_arena {
 };
 
 struct act_entry {       // quantized copy of an activation tensor
-    int kind;            // 1 = q8 (Q8_0 semantics), 2 = q8K
+    int kind;            // 1 = q8 (Q8_0 semantics), 2 = q8K, 3 = q8K in x16 form (act_kind_of)
     q8_act q8;
     q8k_act q8k;
     int64_t K, ncols;
@@ -585,12 +585,47 @@ private:
             e.q8.qs = (int8_t *) c_.scratch.alloc((size_t) (K * ncols));
             e.q8.d = (float *) c_.scratch.alloc((size_t) (K / 32 * ncols) * 4);
             e.q8.s = (int32_t *) c_.scratch.alloc((size_t) (K / 32 * ncols) * 4);
+        } else if (kind == 3) {
+            const size_t size = (size_t) (K / 256 * ((ncols + 15) / 16)) * X16_BYTES;
+            auto it = free_x16_.find(size);
+            if (it != free_x16_.end()) {
+                e.q8k.x16 = it->second;
+                free_x16_.erase(it);
+            } else {
+                e.q8k.x16 = (uint8_t *) c_.scratch.alloc(size);
+            }
         } else {
             e.q8k.qs = (int8_t *) c_.scratch.alloc((size_t) (K * ncols));
             e.q8k.d = (float *) c_.scratch.alloc((size_t) (K / 256 * ncols) * 4);
             e.q8k.bsums = (int16_t *) c_.scratch.alloc((size_t) (K / 16 * ncols) * 2);
         }
         return e;
+    }
+    // a product of several columns with K-quant weights: the matrix-core kernel (launch_mm_kq), which
+    // reads the x16 form
+    static bool kq_multi(const ggml_tensor * mm) {
+        return is_kquant(mm->src[0]->type) && (mm->op == GGML_OP_MUL_MAT_ID ? mm->src[2]->ne[1] : mm->src[1]->ne[1]) >= 2;
+    }
+    // the quantized form of its activation that a mul_mat / mul_mat_id reads (act_entry::kind; 0: none)
+    static int act_kind_of(const ggml_tensor * mm) { return kq_multi(mm) ? 3 : dot_kind(mm->src[0]->type); }
+    // x16 buffers whose readers have all been launched, by size: a later activation may take one (the
+    // stream runs in order), so that a graph's scratch does not grow with its layers
+    std::multimap<size_t, uint8_t *> free_x16_;
+    bool readers_done(int i) const {
+        if (i < 0 || is_output(i)) return false;
+        for (int u : users_[i]) {
+            if (is_view_op(g_->nodes[u]->op) ? !readers_done(u) : !done_[u]) return false;
+        }
+        return true;
+    }
+    void retire_x16(const ggml_tensor * x) {
+        const ggml_tensor * base = x->op == GGML_OP_RESHAPE ? x->src[0] : x;
+        auto it = act_.find(base);
+        if (it == act_.end()) it = act_.find(base = x);
+        if (it == act_.end() || it->second.kind != 3 || !readers_done(node_index(base))) return;
+        const act_entry e = it->second;
+        for (auto k = act_.begin(); k != act_.end();) k = k->second.q8k.x16 == e.q8k.x16 ? act_.erase(k) : std::next(k);
+        free_x16_.insert({ (size_t) (e.K / 256 * ((e.ncols + 15) / 16)) * X16_BYTES, e.q8k.x16 });
     }
     // the quantized form all consumers of node i want (0: none / mixed / not all quantized mul_mats)
     int wanted_act_kind(int i) const {
@@ -599,7 +634,7 @@ private:
         for (int u : users_[i]) {
             const ggml_tensor * n = g_->nodes[u];
             if (n->op != GGML_OP_MUL_MAT || n->src[1] != g_->nodes[i]) return 0;
-            const int k = dot_kind(n->src[0]->type);
+            const int k = act_kind_of(n);
             if (k == 0 || (kind && k != kind)) return 0;
             kind = k;
         }
@@ -607,18 +642,20 @@ private:
     }
 
     // the weight type of the quantized GEMVs that are node u's only consumers (-1: some consumer is
-    // not such a GEMV, or they mix dot types)
-    int gemv_only_consumers(int u) const {
+    // not such a GEMV, or they read different quantized forms); kind: the form they read
+    int gemv_only_consumers(int u, int * kind = nullptr) const {
         if (users_[u].empty()) return -1;
         const ggml_tensor * m = g_->nodes[u];
-        int wtype = -1;
+        int wtype = -1, form = 0;
         for (int j : users_[u]) {
             const ggml_tensor * n = g_->nodes[j];
             if ((n->op != GGML_OP_MUL_MAT && n->op != GGML_OP_MUL_MAT_ID) || n->src[1] != m || n->src[0] == m || attn_.count(j) ||
                 !gemv_capable(n)) return -1;
-            if (wtype >= 0 && dot_kind(n->src[0]->type) != dot_kind(wtype)) return -1;
+            if (wtype >= 0 && act_kind_of(n) != form) return -1;
             wtype = n->src[0]->type;
+            form = act_kind_of(n);
         }
+        if (kind) *kind = form;
         return wtype;
     }
 
@@ -1114,13 +1151,14 @@ private:
                     if (m->ne[1] == rows && norm_deferrable(u, N) && ((uintptr_t) x->data | (uintptr_t) w->data) % 16 == 0) {
                         const gemv_norm nz{ (const float *) x->data, N, (const float *) w->data, eps, 1 };
                         done_[u] = true;
-                        if (max_consumer_rows(u) <= GEMV_PROLOGUE_MAX_ROWS && !gemm_consumer(u) && (rows == 1 || !fuse(FUSE_MC))) {
+                        int kind = 0;
+                        const int wtype = gemv_only_consumers(u, &kind);
+                        if (max_consumer_rows(u) <= GEMV_PROLOGUE_MAX_ROWS && !gemm_consumer(u) && kind != 3 &&
+                            (rows == 1 || !fuse(FUSE_MC))) {
                             norm_[m] = nz;      // every consumer workgroup normalizes for itself
                             return;
                         }
                         // a very wide consumer (the LM head) or a GEMM: normalize and quantize once
-                        const int wtype = gemv_only_consumers(u);
-                        const int kind = dot_kind(wtype);
                         act_entry e = alloc_act(kind, N, rows);
                         gemv_launch L{};
                         L.type = wtype;
@@ -1136,11 +1174,11 @@ private:
                     }
                     const int kind = m->ne[1] == rows ? wanted_act_kind(u) : 0;
                     act_entry e{};
-                    const bool q = (kind == 1 && N % 32 == 0) || (kind == 2 && N % 256 == 0);
+                    const bool q = (kind == 1 && N % 32 == 0) || (kind >= 2 && N % 256 == 0);
                     if (q) e = alloc_act(kind, N, rows);
                     prof_scope ps(this, "rms_norm_mul", (double) (N * rows * 8 + N * 4));
                     launch_rms_norm((const float *) x->data, N, (const float *) w->data, (float *) m->data, N, N, rows, eps,
-                                    q && kind == 1 ? &e.q8 : nullptr, q && kind == 2 ? &e.q8k : nullptr, st_);
+                                    q && kind == 1 ? &e.q8 : nullptr, q && kind >= 2 ? &e.q8k : nullptr, st_);
                     if (q) act_[m] = e;
                     done_[u] = true;
                     wrote_.push_back(m);
@@ -1176,11 +1214,13 @@ private:
         return is_2d_contig(mm);
     }
 
-    // a quantized mul_mat over a prefill-width batch: the int8-MFMA GEMM (same floats as the GEMV)
-    bool gemm_route(const ggml_tensor * mm) const {
+    static bool gemm_wide(const ggml_tensor * mm) {
         const int64_t cols = mm->src[1]->ne[1];
-        const bool wide = cols >= GEMM_MIN_COLS || (cols >= GEMM_WIDE_MIN_COLS && mm->src[0]->ne[1] >= GEMM_WIDE_MIN_ROWS);
-        return mm->op == GGML_OP_MUL_MAT && wide && gemv_capable(mm) &&
+        return cols >= GEMM_MIN_COLS || (cols >= GEMM_WIDE_MIN_COLS && mm->src[0]->ne[1] >= GEMM_WIDE_MIN_ROWS);
+    }
+    // a Q4_0 / Q8_0 mul_mat over a prefill-width batch: the int8-MFMA GEMM (same floats as the GEMV)
+    bool gemm_route(const ggml_tensor * mm) const {
+        return mm->op == GGML_OP_MUL_MAT && gemm_wide(mm) && !is_kquant(mm->src[0]->type) && gemv_capable(mm) &&
                gemm_supported(mm->src[0]->type, mm->src[0]->ne[0], mm->src[0]->ne[1]) &&
                (mm->nb[1] / sizeof(float)) % 4 == 0 && ((uintptr_t) mm->data) % 16 == 0 &&
                (is_repacked(mm->src[0]->type) || ((uintptr_t) mm->src[0]->data) % 16 == 0);
@@ -1194,37 +1234,20 @@ private:
         ggml_tensor * n = g_->nodes[i];
         const ggml_tensor * w = n->src[0];
         const ggml_tensor * x = n->src[1];
-        const int kind = dot_kind(w->type);
-        const act_entry * xa = ensure_act(x, kind);
+        const act_entry * xa = ensure_act(x, 1);
         gemm_launch G{};
         G.type = w->type;
         G.K = w->ne[0];
         G.n_rows = w->ne[1];
         G.ncols = x->ne[1];
-        if (kind == 2) {
-            if (w->type == GGML_TYPE_Q6_K) {
-                const planes p = planes_of(w);
-                G.w = p.qs + p.first_block * 128;
-                G.wqh = p.qh + p.first_block * 64;
-                G.wsc = p.sc + p.first_block * 16;
-                G.wd = p.d + p.first_block;
-            } else {
-                G.w = (const uint8_t *) w->data;
-            }
-            G.xq = xa->q8k.qs;
-            G.xd = xa->q8k.d;
-            G.xbs = xa->q8k.bsums;
-        } else {
-            const planes p = planes_of(w);
-            G.w = p.qs + p.first_block * qs_bytes_of(w->type);
-            G.wd = p.d + p.first_block;
-            G.xq = xa->q8.qs;
-            G.xd = xa->q8.d;
-        }
+        const planes p = planes_of(w);
+        G.w = p.qs + p.first_block * qs_bytes_of(w->type);
+        G.wd = p.d + p.first_block;
+        G.xq = xa->q8.qs;
+        G.xd = xa->q8.d;
         G.y = (float *) n->data;
         G.y_stride = (int64_t) (n->nb[1] / sizeof(float));
-        const double act_bytes = kind == 2 ? 1.0 + 4.0 / 256 + 2.0 / 16 : 1.0 + 4.0 / 32;
-        double bytes = (double) ggml_nbytes(w) + (double) (G.K * G.ncols) * act_bytes + (double) (G.n_rows * G.ncols * 4);
+        double bytes = (double) ggml_nbytes(w) + (double) (G.K * G.ncols) * (1.0 + 4.0 / 32) + (double) (G.n_rows * G.ncols * 4);
         ggml_tensor * written = n;
         const int u = fuse(FUSE_ADD) ? sole_user(i) : -1;
         if (u >= 0) {
@@ -1300,7 +1323,7 @@ private:
                     }
                 }
                 if (kq && !other) {
-                    act_entry e = alloc_act(2, m->ne[0], m->ne[1]);
+                    act_entry e = alloc_act(m->ne[1] >= 2 ? 3 : 2, m->ne[0], m->ne[1]);
                     q8k = e.q8k;
                     for (const ggml_tensor * r : readers) act_[r] = e;
                 }
@@ -1317,11 +1340,11 @@ private:
 
     // Columns per grouped workgroup: about the columns an active expert gets with uniform routing
     // (1 - (1 - k/E)^T of the experts are active), as a power of two in [2, 16]
-    static int moe_cols_per_item(int n_slots, int n_tok, int n_experts) {
+    static int moe_cols_per_item(int n_slots, int n_tok, int n_experts, int most) {
         const double active = n_experts * (1.0 - std::pow(1.0 - std::min(1.0, (double) n_slots / n_experts), (double) n_tok));
         const double avg = (double) n_slots * n_tok / std::max(1.0, active);
         int nc = 2;
-        while (nc < GEMV_MC_MAX_COLS && nc < avg) nc *= 2;
+        while (nc < most && nc < avg) nc *= 2;
         return nc;
     }
 
@@ -1340,14 +1363,15 @@ private:
         return k;
     }
 
-    // The columns of a mul_mat_id grouped by expert (once per ids tensor and graph compute)
-    std::unordered_map<const ggml_tensor *, expert_groups> groups_;
-    const expert_groups & expert_groups_of(const ggml_tensor * ids, int n_experts) {
-        auto it = groups_.find(ids);
+    // The columns of a mul_mat_id grouped by expert, in items of up to nc columns (once per ids tensor,
+    // nc and graph compute)
+    std::map<std::pair<const ggml_tensor *, int>, expert_groups> groups_;
+    const expert_groups & expert_groups_of(const ggml_tensor * ids, int n_experts, int nc, int wtype) {
+        auto it = groups_.find({ ids, nc });
         if (it != groups_.end()) return it->second;
         const int n_slots = (int) ids->ne[0], n_tok = (int) ids->ne[1], ncol = n_slots * n_tok;
         expert_groups g{};
-        g.nc = moe_cols_per_item(n_slots, n_tok, n_experts);
+        g.nc = nc;
         g.max_items = std::min(n_experts, ncol) + (ncol + g.nc - 1) / g.nc;
         g.count = (int32_t *) c_.scratch.alloc((size_t) n_experts * sizeof(int32_t));
         g.offset = (int32_t *) c_.scratch.alloc((size_t) n_experts * sizeof(int32_t));
@@ -1355,10 +1379,10 @@ private:
         g.items = (int32_t *) c_.scratch.alloc((size_t) g.max_items * 3 * sizeof(int32_t));
         g.n_items = (int32_t *) c_.scratch.alloc(sizeof(int32_t));
         {
-            prof_scope ps(this, "moe_group", 0);
+            prof_scope ps(this, wtype == GGML_TYPE_Q5_K || wtype == GGML_TYPE_Q6_K ? "moe_group_k56" : "moe_group", 0);
             launch_moe_group((const int32_t *) ids->data, (int64_t) (ids->nb[1] / sizeof(int32_t)), n_slots, n_tok, n_experts, g, st_);
         }
-        return groups_[ids] = g;
+        return groups_[{ ids, nc }] = g;
     }
 
     // Whether the GEMVs of a group read activation x (f32, not yet quantized) straight from memory,
@@ -1373,6 +1397,13 @@ private:
         int64_t rows = 0;
         for (int j : group) rows += g_->nodes[j]->src[0]->ne[1];
         return rows <= GEMV_PROLOGUE_MAX_ROWS;
+    }
+
+    // profile name of a prefill-width K-quant product (with its workgroup tile, e.g. gemm_q4_K_2x2);
+    // empty for the others, which keep the GEMV names
+    std::string kq_name(const gemv_launch & L, bool wide, const expert_groups * G) const {
+        if (!wide || !is_kquant(L.type)) return {};
+        return std::string("gemm_") + ggml_type_name((enum ggml_type) L.type) + "_" + mm_shape_name(mm_shape_of(L, G));
     }
 
     // quantized GEMV for node i, grouped with the other pending mul_mats that read the same input
@@ -1407,8 +1438,9 @@ private:
         }
 
         // SwiGLU pair inside the group: gate -> silu -> mul(silu, up)
+        const bool kq = kq_multi(n);
         int gate = -1, up = -1, mulnode = -1;
-        if (fuse(FUSE_SWIGLU) && group.size() >= 2 && K <= gemv_swiglu_max_k(wtype)) {
+        if (fuse(FUSE_SWIGLU) && group.size() >= 2 && !kq && K <= gemv_swiglu_max_k(wtype)) {
             for (int a : group) {
                 const int s = sole_user(a);
                 if (s < 0) continue;
@@ -1426,16 +1458,17 @@ private:
             }
         }
 
-        const int kind = dot_kind(wtype);
+        const int kind = act_kind_of(n);
         // several columns (tokens) per workgroup: the activation is quantized once, up front
         const int64_t n_tok = by_id ? ids->ne[1] : ncols;
-        const int mc_nc = by_id ? moe_cols_per_item((int) ids->ne[0], (int) n_tok, (int) n->src[0]->ne[2]) : 0;
-        const bool mc = fuse(FUSE_MC) && n_tok >= 2 && gemv_mc_fits(wtype, (int) K, false, mc_nc) &&
+        const int mc_nc = by_id ? moe_cols_per_item((int) ids->ne[0], (int) n_tok, (int) n->src[0]->ne[2],
+                                                    kq ? MOE_GROUP_MAX_COLS : GEMV_MC_MAX_COLS) : 0;
+        const bool mc = !kq && fuse(FUSE_MC) && n_tok >= 2 && gemv_mc_fits(wtype, (int) K, false, mc_nc) &&
                         (gate < 0 || gemv_mc_fits(wtype, (int) K, true, mc_nc));
         const auto nz = norm_.find(x);
         gemv_norm pro{};
         const act_entry * xa = nullptr;
-        if (mc) {
+        if (mc || kq) {
             if (act_.count(x) && act_.at(x).kind == kind) {
                 xa = &act_.at(x);
             } else if (nz != norm_.end() && K <= act_quant_max_k(wtype, nz->second.rms != 0)) {
@@ -1522,6 +1555,7 @@ private:
         L.K = (int) K;
         L.ncols = (int) ncols;
         if (!xa) L.norm = pro;
+        else if (kind == 3) L.xq = (const int8_t *) xa->q8k.x16;
         else if (kind == 1) { L.xq = xa->q8.qs; L.xd = xa->q8.d; L.xs = xa->q8.s; }
         else { L.xq = xa->q8k.qs; L.xd = xa->q8k.d; L.xbs = xa->q8k.bsums; }
         if (by_id) {
@@ -1557,11 +1591,9 @@ private:
         if (by_id && c_.timing && !route_in) n_unique_experts = distinct_ids(ids, n->src[0]->ne[2]);
         const double x_bytes = (double) (K * ggml_nrows(x) * 4) + (xa ? 0.0 : (double) (K * 4));
         // one column per workgroup, or several (mul_mat_id: the tokens routed to each expert)
-        const expert_groups * G = mc && by_id ? &expert_groups_of(ids, (int) n->src[0]->ne[2]) : nullptr;
+        const expert_groups * G = (mc || kq) && by_id ? &expert_groups_of(ids, (int) n->src[0]->ne[2], mc_nc, wtype) : nullptr;
         auto run = [&](const gemv_launch & X) {
-            // GGML_HIP_NO_MFMA_GEMV: the multi-column GEMV for every such launch (comparisons)
-            static const bool no_mfma = getenv("GGML_HIP_NO_MFMA_GEMV") != nullptr;
-            if (mc && !G && !no_mfma && gemv_mfma_supported(X)) launch_gemv_mfma(X, st_);
+            if (kq) launch_mm_kq(X, G, st_);
             else if (mc) launch_gemv_mc(X, G, G ? (int) n_tok : X.ncols, st_);
             else launch_gemv(X, st_);
         };
@@ -1624,10 +1656,12 @@ private:
         L.n_mats = (int) group.size();
         for (size_t k = 0; k < group.size(); k++) fill_mat(L.m[k], group[k], bytes, true);
         {
-            prof_scope ps(this, gemv_prof_name(wtype, false), bytes);
+            const std::string gname = kq_name(L, !by_id && gemm_wide(n), G);
+            prof_scope ps(this, !gname.empty() ? gname.c_str() : gemv_prof_name(wtype, false), bytes);
             run(L);
         }
         for (int j : group) done_[j] = true;
+        if (kq) retire_x16(x);
     }
 
     // silu(gate) -> mul(., up) on f32 2-D views (prefill: the fused gate/up projection's halves, or
@@ -1636,6 +1670,13 @@ private:
     static bool disjoint_or_same(const ggml_tensor * a, const ggml_tensor * b) {
         const uint8_t * a0 = (const uint8_t *) a->data, * b0 = (const uint8_t *) b->data;
         return a0 == b0 || a0 + ggml_nbytes(a) <= b0 || b0 + ggml_nbytes(b) <= a0;
+    }
+    // a view of t's rows as one 2-D matrix (its rows evenly strided)
+    static tview rows_2d(const ggml_tensor * t) {
+        tview v = tv(t);
+        v.ne[1] = ggml_nrows(t);
+        v.ne[2] = v.ne[3] = 1;
+        return v;
     }
     bool op_swiglu(int i) {
         ggml_tensor * sn = g_->nodes[i];
@@ -1646,7 +1687,9 @@ private:
         const ggml_tensor * gt = sn->src[0], * up = mn->src[1];
         if (mn->op != GGML_OP_MUL || mn->src[0] != sn || !ggml_are_same_shape(gt, mn) || !ggml_are_same_shape(up, mn)) return false;
         for (const ggml_tensor * t : { gt, up, (const ggml_tensor *) mn }) {
-            if (t->type != GGML_TYPE_F32 || t->nb[0] != sizeof(float) || t->ne[2] != 1 || t->ne[3] != 1) return false;
+            // rows evenly strided (several tokens' expert slots: [n_ff, slots, tokens])
+            if (t->type != GGML_TYPE_F32 || t->nb[0] != sizeof(float) || t->ne[3] != 1 ||
+                (t->ne[2] != 1 && t->nb[2] != t->nb[1] * t->ne[1])) return false;
         }
         // the kernel reads gate[i] and up[i] before writing out[i]: the output may sit exactly on
         // either input, never across one (gate is not an input of the mul, so the allocator may
@@ -1671,14 +1714,16 @@ private:
         const ggml_tensor * gt = g_->nodes[i]->src[0];
         ggml_tensor * mn = g_->nodes[mj];
         const ggml_tensor * up = mn->src[1];
-        const int64_t K = mn->ne[0], ncols = mn->ne[1];
-        const int want = is_2d_contig(mn) ? wanted_act_kind(mj) : 0;
-        const int kind = (want == 1 && K % 32 == 0) || (want == 2 && K % 256 == 0) ? want : 0;
+        const int64_t K = mn->ne[0], ncols = ggml_nrows(mn);
+        int want = 0;
+        if (!fuse(FUSE_ACTQ) || !ggml_is_contiguous(mn) || gemv_only_consumers(mj, &want) < 0) want = 0;
+        const int kind = (want == 1 && K % 32 == 0) || (want >= 2 && K % 256 == 0) ? want : 0;
         act_entry e{};
         if (kind) e = alloc_act(kind, K, ncols);
         {
             prof_scope ps(this, "swiglu", (double) (K * ncols * 12));
-            launch_swiglu(tv(gt), tv(up), tv(mn), kind == 1 ? &e.q8 : nullptr, kind == 2 ? &e.q8k : nullptr, st_);
+            launch_swiglu(rows_2d(gt), rows_2d(up), rows_2d(mn), kind == 1 ? &e.q8 : nullptr, kind >= 2 ? &e.q8k : nullptr,
+                          !kind || is_output(mj) || c_.cb, st_);
         }
         if (kind) act_[mn] = e;
         done_[mj] = true;
@@ -1791,7 +1836,7 @@ private:
             if (m->op != GGML_OP_MUL || m->src[0] != n || w->type != GGML_TYPE_F32 || ggml_nrows(w) != 1 || w->ne[0] != x->ne[0] ||
                 !ggml_is_contiguous(w) || !ggml_is_contiguous(m) || m->ne[1] != ggml_nrows(x) ||
                 ((uintptr_t) x->data | (uintptr_t) w->data) % 16) continue;
-            if (!norm_deferrable(u, x->ne[0]) || wanted_act_kind(u) != 2) continue;
+            if (!norm_deferrable(u, x->ne[0]) || wanted_act_kind(u) != 3) continue;
             nn = j;
             nm = u;
             memcpy(&eps, n->op_params, 4);
@@ -1862,7 +1907,7 @@ private:
             // the next rms_norm * w, normalized and quantized in the same launch (what op_rms_norm
             // would do in an act_quant launch of its own)
             ggml_tensor * mn = g_->nodes[nm];
-            act_entry e = alloc_act(2, n_embd, T);
+            act_entry e = alloc_act(3, n_embd, T);
             {
                 prof_scope ps(this, "moe_wsum_q8k", wsum_bytes + (double) (n_embd * 4 + n_embd * T + (n_embd / 256 * 4 + n_embd / 16 * 2) * T));
                 launch_wsum_norm_q8k(M, (const float *) mn->src[1]->data, eps, e.q8k, st_);
@@ -1955,7 +2000,7 @@ private:
             A.out = A0.out + (int64_t) q0 * A0.out_nb1;
             const int64_t K = (int64_t) A0.n_head * A0.hd;
             if (A0.out_q.qs) A.out_q = q8_act{ A0.out_q.qs + q0 * K, A0.out_q.d + q0 * (K / 32), A0.out_q.s + q0 * (K / 32) };
-            if (A0.out_q8k.qs) A.out_q8k = q8k_act{ A0.out_q8k.qs + q0 * K, A0.out_q8k.d + q0 * (K / 256), A0.out_q8k.bsums + q0 * (K / 16) };
+            if (A0.out_q8k.set()) A.out_q8k.x16 = A0.out_q8k.x16 + (q0 / 16) * (K / 256) * X16_BYTES;
             launch_attn_decode(A, st_);
         }
     }
@@ -1987,8 +2032,8 @@ private:
             act_entry e = alloc_act(1, ctn->ne[0], n_q);
             A.out_q = e.q8;
             act_[ctn] = e;
-        } else if (kind == 2 && (A.n_head * A.hd) % 256 == 0 && 256 % A.hd == 0) {
-            act_entry e = alloc_act(2, ctn->ne[0], n_q);
+        } else if (kind >= 2 && (A.n_head * A.hd) % 256 == 0 && 256 % A.hd == 0) {
+            act_entry e = alloc_act(kind, ctn->ne[0], n_q);
             A.out_q8k = e.q8k;
             act_[ctn] = e;
         }

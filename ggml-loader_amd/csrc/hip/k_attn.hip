@@ -580,18 +580,18 @@ __global__ __launch_bounds__(CMB_K_PARTS * 256) void attn_combine_q8k_kernel(con
             const float iscale = -127.f / bval;
             qv = round_half_even(iscale * v);
             qv = qv < 127 ? qv : 127;
-            if (j == 0) A.out_q8k.d[q * nsb + sb] = 1 / iscale;
+            if (j == 0) A.out_q8k.put_d(nsb, q, sb, 1 / iscale);
         } else if (j == 0) {
-            A.out_q8k.d[q * nsb + sb] = 0.0f;
+            A.out_q8k.put_d(nsb, q, sb, 0.0f);
         }
-        A.out_q8k.qs[q * K + (int64_t) sb * 256 + j] = (int8_t) qv;
+        A.out_q8k.put_q(nsb, q, sb, j, qv);
         s_q[j] = qv;
     }
     __syncthreads();
     if (t < 16) {
         int sum = 0;
         for (int i = 0; i < 16; i++) sum += s_q[t * 16 + i];
-        A.out_q8k.bsums[q * (K / 16) + (int64_t) sb * 16 + t] = (int16_t) sum;
+        A.out_q8k.put_sum(nsb, q, sb, t, sum);
     }
 }
 
@@ -1104,12 +1104,12 @@ __global__ __launch_bounds__(ATT_THREADS) void attn_pv_mq_kernel(const attn_laun
 template <int HD>
 static void launch_combine(const attn_launch & A, int pv_splits, hipStream_t st) {
     if constexpr (256 % HD == 0) {
-        if (A.out_q8k.qs) {
+        if (A.out_q8k.set()) {
             return launch(attn_combine_q8k_kernel<HD>, dim3(A.n_head * HD / 256, A.n_q), dim3(CMB_K_PARTS * 256), 0, st, A,
                           pv_splits);
         }
     }
-    if (A.out_q8k.qs) HIP_ABORT("attn: a Q8_K output needs 256 %% hd == 0");
+    if (A.out_q8k.set()) HIP_ABORT("attn: a Q8_K output needs 256 %% hd == 0");
     launch(attn_combine_kernel<HD>, dim3(A.n_head, A.n_q), dim3(CMB_PARTS * HD), 0, st, A, pv_splits);
 }
 
@@ -1238,8 +1238,8 @@ void launch_attn_decode(const attn_launch & A_in, hipStream_t st) {
     if (A.n_head % A.n_head_kv) HIP_ABORT("attn: n_head %% n_head_kv");
     if (A.scratch_bytes < attn_scratch_bytes(A.n_kv, A.n_q, A.n_head, A.hd)) HIP_ABORT("attn: scratch too small");
     if (A.out_q.qs && (A.hd % 32)) HIP_ABORT("attn: quantized output needs hd %% 32 == 0");
-    if (A.acc && (A.n_q != 1 || A.out_q.qs || A.out_q8k.qs || ((uintptr_t) A.acc) % 16)) HIP_ABORT("attn: the accumulated output takes one query, no quantized copy, 16-byte alignment");
-    if (A.out_q8k.qs && (A.out_q.qs || (A.n_head * A.hd) % 256 || 256 % A.hd)) HIP_ABORT("attn: Q8_K output needs n_head * hd %% 256 == 0 and 256 %% hd == 0");
+    if (A.acc && (A.n_q != 1 || A.out_q.qs || A.out_q8k.set() || ((uintptr_t) A.acc) % 16)) HIP_ABORT("attn: the accumulated output takes one query, no quantized copy, 16-byte alignment");
+    if (A.out_q8k.set() && (A.out_q.qs || (A.n_head * A.hd) % 256 || 256 % A.hd)) HIP_ABORT("attn: Q8_K output needs n_head * hd %% 256 == 0 and 256 %% hd == 0");
     if (A.n_q > ATT_MAX_Q) {
         // many queries: scores and PV on the matrix cores
         switch (A.hd) {

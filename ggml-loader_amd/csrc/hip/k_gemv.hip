@@ -138,8 +138,7 @@ void launch_quantize_q8(const float * x, int64_t x_col_stride, int64_t K, int64_
 // Q8_K (ggml quantize_row_q8_K_ref): max = the value of largest magnitude (first one on ties),
 // iscale = -127/max, q = min(127, nearest_int(iscale*x)), d = 1/iscale, bsums over 16s.
 // One 256-thread block per (super-block, column).
-__global__ void quantize_q8k_kernel(const float * __restrict__ x, int64_t x_col_stride, int64_t K,
-                                    int8_t * __restrict__ qs, float * __restrict__ d, int16_t * __restrict__ bsums) {
+__global__ void quantize_q8k_kernel(const float * __restrict__ x, int64_t x_col_stride, int64_t K, q8k_act out) {
     __shared__ float s_ax[4];
     __shared__ int s_idx[4];
     __shared__ float s_val[4];
@@ -172,23 +171,26 @@ __global__ void quantize_q8k_kernel(const float * __restrict__ x, int64_t x_col_
         const float iscale = -127.f / bval;
         q = round_half_even(iscale * v);
         q = q < 127 ? q : 127;
-        if (t == 0) d[c * nsb + sb] = 1 / iscale;
+        if (t == 0) out.put_d(nsb, c, sb, 1 / iscale);
     } else if (t == 0) {
-        d[c * nsb + sb] = 0.0f;
+        out.put_d(nsb, c, sb, 0.0f);
     }
-    qs[c * K + sb * 256 + t] = (int8_t) q;
+    out.put_q(nsb, c, sb, t, q);
     s_q[t] = q;
     __syncthreads();
     if (t < 16) {
         int sum = 0;
         for (int i = 0; i < 16; i++) sum += s_q[t * 16 + i];
-        bsums[c * (K / 16) + sb * 16 + t] = (int16_t) sum;
+        out.put_sum(nsb, c, sb, t, sum);
     }
 }
 
 void launch_quantize_q8k(const float * x, int64_t x_col_stride, int64_t K, int64_t ncols, q8k_act out, hipStream_t st) {
+    if (out.x16 && q8k_x16_ok(x, x_col_stride, nullptr, 0, nullptr, 0)) {
+        return launch_q8k_x16(x, x_col_stride, nullptr, 0, nullptr, 0, K, ncols, out, st);
+    }
     dim3 grid((unsigned) (K / 256), (unsigned) ncols);
-    launch(quantize_q8k_kernel, grid, dim3(256), 0, st, x, x_col_stride, K, out.qs, out.d, out.bsums);
+    launch(quantize_q8k_kernel, grid, dim3(256), 0, st, x, x_col_stride, K, out);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -534,6 +536,29 @@ __device__ __forceinline__ void stage_x(const gemv_launch & L, int col, const ge
     __syncthreads();
 }
 
+// A staged Q8_K column out to global memory, in the form the output asks for (a workgroup of GEMV_NT
+// threads). x16: a thread gathers the 8 quants 64 q + l, l + 8, ... of a super-block, one unit.
+__device__ __forceinline__ void store_q8k(const gemv_lds & s, int K, int col, const q8k_act & out) {
+    const int nsb = K / 256;
+    if (out.x16) {
+        for (int u = threadIdx.x; u < nsb * 32; u += GEMV_NT) {
+            const int sb = u / 32, l = u / 4 % 8, q = u % 4;
+            const int8_t * x = s.xq + sb * 256 + 64 * q + l;
+            __half v[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) v[k] = __int2half_rn(x[8 * k]);
+            uint4 o;
+            memcpy(&o, v, 16);
+            *(uint4 *) out.unit(nsb, col, sb, 4 * l + q) = o;
+        }
+    } else {
+        int8_t * qs = out.qs + (int64_t) col * K;
+        for (int i = threadIdx.x * 16; i < K; i += GEMV_NT * 16) *(int4 *) (qs + i) = *(const int4 *) (s.xq + i);
+    }
+    for (int i = threadIdx.x; i < nsb; i += GEMV_NT) out.put_d(nsb, col, i, s.xd[i]);
+    for (int i = threadIdx.x; i < nsb * 16; i += GEMV_NT) out.put_sum(nsb, col, i / 16, i % 16, s.xbs[i]);
+}
+
 // The prologue run once per column into global memory, for consumers too wide to redo it in every
 // workgroup (the LM head): same arithmetic, so the GEMV that copies the result computes the same floats.
 template <int TYPE>
@@ -548,12 +573,11 @@ __global__ __launch_bounds__(GEMV_NT) void act_quant_kernel(const gemv_launch L,
     prologue_load<TYPE, true>(L, col, xv, wv);
     prologue_finish<TYPE>(L, col, xv, wv, s, s_red);
     __syncthreads();
-    int8_t * qs = (TYPE == GGML_TYPE_Q4_K ? q8k.qs : q8.qs) + (int64_t) col * K;
-    for (int i = threadIdx.x * 16; i < K; i += GEMV_NT * 16) *(int4 *) (qs + i) = *(const int4 *) (s.xq + i);
     if (TYPE == GGML_TYPE_Q4_K) {
-        for (int i = threadIdx.x; i < K / 256; i += GEMV_NT) q8k.d[(int64_t) col * (K / 256) + i] = s.xd[i];
-        for (int i = threadIdx.x; i < K / 16; i += GEMV_NT) q8k.bsums[(int64_t) col * (K / 16) + i] = s.xbs[i];
+        store_q8k(s, K, col, q8k);
     } else {
+        int8_t * qs = q8.qs + (int64_t) col * K;
+        for (int i = threadIdx.x * 16; i < K; i += GEMV_NT * 16) *(int4 *) (qs + i) = *(const int4 *) (s.xq + i);
         for (int i = threadIdx.x; i < K / 32; i += GEMV_NT) {
             q8.d[(int64_t) col * (K / 32) + i] = s.xd[i];
             q8.s[(int64_t) col * (K / 32) + i] = s.xs[i];
@@ -655,10 +679,7 @@ __global__ __launch_bounds__(GEMV_NT) void wsum_norm_q8k_kernel(const moe_wsum M
     }
     quant_chunk<GGML_TYPE_Q4_K, 16>(x0, t, t < nchunk, s);
     __syncthreads();
-    int8_t * qs = q8k.qs + (int64_t) tok * K;
-    for (int i = t * 16; i < K; i += GEMV_NT * 16) *(int4 *) (qs + i) = *(const int4 *) (s.xq + i);
-    for (int i = t; i < K / 256; i += GEMV_NT) q8k.d[(int64_t) tok * (K / 256) + i] = s.xd[i];
-    for (int i = t; i < K / 16; i += GEMV_NT) q8k.bsums[(int64_t) tok * (K / 16) + i] = s.xbs[i];
+    store_q8k(s, K, tok, q8k);
 }
 
 bool wsum_norm_q8k_supported(const moe_wsum & M, const float * nw) {

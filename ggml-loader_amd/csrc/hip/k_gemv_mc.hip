@@ -1,12 +1,12 @@
 // k_gemv_mc.hip — quantized GEMV over several activation columns per workgroup: each weight row
 // block is read once for up to GEMV_MC_MAX_COLS columns (multi-token decode steps, prompts too
-// short for the GEMM, Q4_K prompts) and, for ggml_mul_mat_id, once for all the tokens routed to
+// short for the GEMM) and, for ggml_mul_mat_id, once for all the tokens routed to
 // its expert — the batched expert grouping of the reference's MoE engine (build_prefill_lists /
 // matmul_batch, qwen_model.c:742-772, 862-939), here over the expert lists that moe_group_kernel
 // builds on the device from the routing ids.
 //
 // Per (row, column) the arithmetic is k_gemv.hip's: the same integer block dots against the
-// pre-quantized activation (Q8_0 / Q8_K), the same float terms, added in block order by one
+// pre-quantized Q8_0 activation, the same float terms, added in block order by one
 // thread per (row, column[, gate/up]) chain, so the result is the CPU reference's float.
 #include "gemv_mc_impl.h"
 
@@ -21,7 +21,6 @@ static bool launch_mc_dispatch(const gemv_launch & L, const expert_groups * G, i
     switch (L.type) {
         case GGML_TYPE_Q4_0: return launch_mc_q4_0(SWIGLU, L, G, max_cols, st, dry);
         case GGML_TYPE_Q8_0: return launch_mc_q8_0(SWIGLU, L, G, max_cols, st, dry);
-        case GGML_TYPE_Q4_K: return launch_mc_q4_k(SWIGLU, L, G, max_cols, st, dry);
         default: return false;
     }
 }
@@ -115,7 +114,7 @@ __global__ __launch_bounds__(256) void moe_group_kernel(const int32_t * ids, int
 
 bool gemv_mc_supported(const gemv_launch & L, int max_cols) {
     if (L.norm.x || !L.xq || L.ncols < 1 || max_cols < 1) return false;
-    if (L.type == GGML_TYPE_Q4_K ? L.K % 256 != 0 : L.K % 32 != 0) return false;
+    if (L.K % 32 != 0) return false;
     return L.swiglu ? launch_mc_dispatch<true>(L, nullptr, max_cols, nullptr, true)
                     : launch_mc_dispatch<false>(L, nullptr, max_cols, nullptr, true);
 }
@@ -128,7 +127,7 @@ bool gemv_mc_fits(int type, int K, bool swiglu, int nc) {
     L.n_mats = swiglu ? 2 : 1;
     L.swiglu = swiglu;
     L.xq = (const int8_t *) &L;   // any non-null pointer: nothing is launched
-    if (type == GGML_TYPE_Q4_K ? K % 256 != 0 : K % 32 != 0) return false;
+    if (K % 32 != 0) return false;
     expert_groups g{};
     g.nc = nc;
     const expert_groups * G = nc > 0 ? &g : nullptr;
@@ -150,7 +149,7 @@ void launch_moe_group(const int32_t * ids, int64_t ids_stride, int n_slots, int 
                       hipStream_t st) {
     if (n_experts < 1 || n_experts > 4096 || n_slots < 1 || n_tok < 1) HIP_ABORT("moe_group: %d experts", n_experts);
     const int ncol = n_slots * n_tok;
-    if (g.nc < 1 || g.nc > GEMV_MC_MAX_COLS || g.max_items < std::min(n_experts, ncol) + (ncol + g.nc - 1) / g.nc) {
+    if (g.nc < 1 || g.nc > MOE_GROUP_MAX_COLS || g.max_items < std::min(n_experts, ncol) + (ncol + g.nc - 1) / g.nc) {
         HIP_ABORT("moe_group: %d items of %d columns cannot hold %d columns", g.max_items, g.nc, ncol);
     }
     launch(moe_group_kernel, dim3(1), dim3(256), (size_t) n_experts * 2 * sizeof(int), st, ids, ids_stride, n_slots, n_tok,

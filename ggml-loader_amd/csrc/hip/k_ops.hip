@@ -21,9 +21,9 @@ static unsigned grid1(int64_t n, int threads) { return (unsigned) ((n + threads 
 // Q8_K quantization (ggml quantize_row_q8_K_ref) of one 256-element super-block held one value per
 // thread of a 256-thread block: the value of largest magnitude (lowest index on ties) sets
 // iscale = -127 / max, q = min(127, round-half-even(iscale * o)), d = 1 / iscale (0 for an all-zero
-// block), bsums = sums of 16 consecutive q. qs, d and bsums point at the super-block's entries.
+// block), bsums = sums of 16 consecutive q; written as super-block sb of column col of out.
 // Every thread of the block must call it (it synchronizes the block).
-__device__ void q8k_superblock(float o, int t, int8_t * qs, float * d, int16_t * bsums) {
+__device__ void q8k_superblock(float o, int t, const q8k_act & out, int64_t nsb, int64_t col, int64_t sb) {
     __shared__ float s_fx[4];
     __shared__ int s_ix[4];
     __shared__ float s_vx[4];
@@ -50,13 +50,13 @@ __device__ void q8k_superblock(float o, int t, int8_t * qs, float * d, int16_t *
         const float iscale = -127.f / bval;
         q = round_half_even(iscale * o);
         q = q < 127 ? q : 127;
-        if (t == 0) *d = 1 / iscale;
+        if (t == 0) out.put_d(nsb, col, sb, 1 / iscale);
     } else if (t == 0) {
-        *d = 0.0f;
+        out.put_d(nsb, col, sb, 0.0f);
     }
-    qs[t] = (int8_t) q;
+    out.put_q(nsb, col, sb, t, q);
     const float bs = group_sum<16>((float) q);
-    if ((t % 16) == 0) bsums[t / 16] = (int16_t) bs;
+    if ((t % 16) == 0) out.put_sum(nsb, col, sb, t / 16, (int) bs);
 }
 
 // One 256-thread block per row; each thread holds its EPT elements (i = it*256 + t) in registers,
@@ -111,8 +111,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const float * __restrict_
             }
         } else if (QUANT == 2) {
             // one super-block of 256 per iteration (n % 256 == 0)
-            q8k_superblock(o, t, q8k.qs + row * n + (int64_t) it * 256, q8k.d + row * (n / 256) + it,
-                           q8k.bsums + row * (n / 16) + (int64_t) it * 16);
+            q8k_superblock(o, t, q8k, n / 256, row, it);
         }
     }
 }
@@ -371,10 +370,9 @@ __global__ __launch_bounds__(256) void swiglu_kernel(tview g, tview u, tview d, 
         v = y * *(const float *) at(u, i, c, 0, 0);
         *(float *) at(d, i, c, 0, 0) = v;
     }
-    if (qk.qs) {
+    if (qk.set()) {
         // K % 256 == 0: every thread holds an element
-        q8k_superblock(v, threadIdx.x, qk.qs + c * K + (int64_t) blockIdx.x * 256, qk.d + c * (K / 256) + blockIdx.x,
-                       qk.bsums + c * (K / 16) + (int64_t) blockIdx.x * 16);
+        q8k_superblock(v, threadIdx.x, qk, K / 256, c, blockIdx.x);
         return;
     }
     if (!q.qs) return;
@@ -393,12 +391,17 @@ __global__ __launch_bounds__(256) void swiglu_kernel(tview g, tview u, tview d, 
     }
 }
 
-void launch_swiglu(const tview & gate, const tview & up, const tview & dst, const q8_act * q, const q8k_act * qk, hipStream_t st) {
+void launch_swiglu(const tview & gate, const tview & up, const tview & dst, const q8_act * q, const q8k_act * qk, bool keep, hipStream_t st) {
     if (dst.ne[2] != 1 || dst.ne[3] != 1 || (q && dst.ne[0] % 32) || (qk && dst.ne[0] % 256) || (q && qk)) {
         HIP_ABORT("swiglu: unsupported shape");
     }
     const q8_act none{};
     const q8k_act nonek{};
+    if (qk && qk->x16 && gate.nb[1] % 4 == 0 && up.nb[1] % 4 == 0 && dst.nb[1] % 4 == 0 &&
+        q8k_x16_ok((const float *) gate.data, gate.nb[1] / 4, (const float *) up.data, up.nb[1] / 4, (const float *) dst.data, dst.nb[1] / 4)) {
+        return launch_q8k_x16((const float *) gate.data, gate.nb[1] / 4, (const float *) up.data, up.nb[1] / 4,
+                              keep ? (float *) dst.data : nullptr, dst.nb[1] / 4, dst.ne[0], dst.ne[1], *qk, st);
+    }
     launch(swiglu_kernel, dim3((unsigned) ((dst.ne[0] + 255) / 256), (unsigned) dst.ne[1]), dim3(256), 0, st, gate, up, dst,
            q ? *q : none, qk ? *qk : nonek);
 }
@@ -1058,12 +1061,9 @@ __global__ __launch_bounds__(256) void mul_mat_rows_norm_kernel(tview w, const f
     __syncthreads();
     // the normalized column's Q8_K form for the norm's quantized consumers (q8k set): workgroup x
     // quantizes super-blocks x, x + gridDim.x, ... (every workgroup holds the whole column)
-    if (q8k.qs) {
+    if (q8k.set()) {
         const int64_t nsb = K / 256;
-        for (int64_t sb = blockIdx.x; sb < nsb; sb += gridDim.x) {
-            q8k_superblock(s_y[sb * 256 + t], t, q8k.qs + col * K + sb * 256, q8k.d + col * nsb + sb,
-                           q8k.bsums + col * (K / 16) + sb * 16);
-        }
+        for (int64_t sb = blockIdx.x; sb < nsb; sb += gridDim.x) q8k_superblock(s_y[sb * 256 + t], t, q8k, nsb, col, sb);
     }
     if (o >= w.ne[1]) return;
     double acc = 0.0;
@@ -1106,7 +1106,7 @@ bool mul_mat_rows_norm_supported(const tview & w, int64_t K) {
 void launch_mul_mat_rows_norm(const tview & w, const float * x, int64_t x_stride, const float * nw, float eps, float * y_out,
                               int64_t y_stride, const tview & dst, int64_t ncols, q8k_act q8k, hipStream_t st) {
     if (!mul_mat_rows_norm_supported(w, w.ne[0]) || dst.ne[0] != w.ne[1] || dst.ne[1] != ncols || dst.nb[0] != 4 ||
-        (q8k.qs && w.ne[0] % 256)) {
+        (q8k.set() && w.ne[0] % 256)) {
         HIP_ABORT("mul_mat_rows_norm: unsupported operands");
     }
     launch(mul_mat_rows_norm_kernel, dim3((unsigned) ((w.ne[1] + 3) / 4), (unsigned) ncols), dim3(256),

@@ -71,10 +71,44 @@ void launch_unpack_q6k(uint8_t * raw, q6k_planes p, int64_t nblocks, int64_t fir
 // ---------------------------------------------------------------------------------------------
 // activation quantization of ncols columns of K floats (column c at x + c*x_col_stride floats)
 struct q8_act { int8_t * qs; float * d; int32_t * s; };     // Q8_0 semantics, per-column K / K/32 / K/32
-struct q8k_act { int8_t * qs; float * d; int16_t * bsums; }; // Q8_K semantics, per-column K / K/256 / K/16
+// Q8_K semantics: per column K int8, K/256 d and K/16 sums (the GEMVs of one column), or x16 (the
+// multi-column products on the matrix cores, mm_kq_impl.h): for every group of 16 columns and every
+// super-block X16_BYTES bytes of 16-byte units [unit][column of the group]. The quants are f16, with
+// element 8k + l (slice l) in unit 4 l + k / 8 at k % 8, so that the operand of slice l is 1 KB in
+// lane order; units 32 and 33 hold the 16 sums as f16, unit 34 d; unit 35 pads a group to nine 1 KB
+// pieces. The group's columns past the last one are never written, and only reach outputs that no
+// one stores.
+constexpr int X16_PIECES = 9, X16_BYTES = X16_PIECES * 1024, X16_USED = 35, X16_SUMS = 32 * 256, X16_D = 34 * 256;
+struct q8k_act {
+    int8_t * qs; float * d; int16_t * bsums;
+    uint8_t * x16;
+    __host__ __device__ __forceinline__ bool set() const { return qs || x16; }
+    // unit u of super-block sb of a column of nsb super-blocks
+    __device__ __forceinline__ uint8_t * unit(int64_t nsb, int64_t col, int64_t sb, int u) const {
+        return x16 + ((col / 16) * nsb + sb) * X16_BYTES + u * 256 + (col % 16) * 16;
+    }
+    // quant e of super-block sb of the column; its scale; the sum of its group g
+    __device__ __forceinline__ void put_q(int64_t nsb, int64_t col, int64_t sb, int e, int q) const {
+        if (x16) ((__half *) unit(nsb, col, sb, e % 8 * 4 + e / 64))[e / 8 % 8] = __int2half_rn(q);
+        else qs[(col * nsb + sb) * 256 + e] = (int8_t) q;
+    }
+    __device__ __forceinline__ void put_d(int64_t nsb, int64_t col, int64_t sb, float v) const {
+        if (x16) *(float *) unit(nsb, col, sb, 34) = v;
+        else d[col * nsb + sb] = v;
+    }
+    __device__ __forceinline__ void put_sum(int64_t nsb, int64_t col, int64_t sb, int g, int v) const {
+        if (x16) ((__half *) unit(nsb, col, sb, 32 + g / 8))[g % 8] = __int2half_rn(v);
+        else bsums[(col * nsb + sb) * 16 + g] = (int16_t) v;
+    }
+};
 
 void launch_quantize_q8(const float * x, int64_t x_col_stride, int64_t K, int64_t ncols, q8_act out, hipStream_t st);
 void launch_quantize_q8k(const float * x, int64_t x_col_stride, int64_t K, int64_t ncols, q8k_act out, hipStream_t st);
+// columns of a, or of silu(a) * b (b not null; its floats then also to y, if not null), to the x16 form:
+// K a multiple of 256, every column 16-byte aligned (q8k_x16_ok)
+bool q8k_x16_ok(const float * a, int64_t a_stride, const float * b, int64_t b_stride, const float * y, int64_t y_stride);
+void launch_q8k_x16(const float * a, int64_t a_stride, const float * b, int64_t b_stride, float * y, int64_t y_stride, int64_t K,
+                    int64_t ncols, q8k_act out, hipStream_t st);
 
 // ---------------------------------------------------------------------------------------------
 // quantized GEMV / small-batch GEMM: y[c][r] = W[r] . x[c] (+ add[c][r]) for up to 4 weight
@@ -101,8 +135,7 @@ struct gemv_mat {
 
 // ---------------------------------------------------------------------------------------------
 // prefill GEMM on the matrix cores: y[c][r] = W[r] . x[c] (+ add[c][r]) for Q4_0 / Q8_0 weights
-// in the plane layout with Q8_0-quantized activation columns, or Q4_K weights (ggml blocks) with
-// Q8_K-quantized columns; the same floats as the GEMV.
+// in the plane layout with Q8_0-quantized activation columns; the same floats as the GEMV.
 constexpr int GEMM_MIN_COLS = 64;   // narrower products stay on the GEMV, except:
 // an output projection this tall (an LM head) takes the GEMM from GEMM_WIDE_MIN_COLS columns: its
 // weights stream once at the GEMM's rate, where the multi-column GEMV would stage every column's
@@ -111,17 +144,14 @@ constexpr int GEMM_WIDE_MIN_COLS = 16;
 constexpr int64_t GEMM_WIDE_MIN_ROWS = 65536;
 
 struct gemm_launch {
-    int             type;      // GGML_TYPE_Q4_0 / Q8_0 / Q4_K / Q5_K / Q6_K
-    int64_t         K;         // row length (a multiple of 128; of 256 for the K-quants)
+    int             type;      // GGML_TYPE_Q4_0 / Q8_0
+    int64_t         K;         // row length (a multiple of 128)
     int64_t         n_rows;
     int64_t         ncols;
-    const uint8_t * w;         // Q4_0 / Q8_0: qs plane of row 0; Q4_K / Q5_K: row 0's first block; Q6_K: its low-bit plane
-    const __half *  wd;        // Q4_0 / Q8_0 / Q6_K: d plane of row 0
-    const uint8_t * wqh;       // Q6_K: high-bit plane of row 0 (64 bytes per block)
-    const int8_t *  wsc;       // Q6_K: scale plane of row 0 (16 per block)
+    const uint8_t * w;         // qs plane of row 0
+    const __half *  wd;        // d plane of row 0
     const int8_t *  xq;        // activation column c at xq + c * K
-    const float *   xd;        // and its scales at xd + c * K / 32 (Q8_0) or xd + c * K / 256 (Q8_K)
-    const int16_t * xbs;       // Q8_K: the column's 16-element sums at xbs + c * K / 16
+    const float *   xd;        // and its scales at xd + c * K / 32
     float *         y;         // output column c at y + c * y_stride
     int64_t         y_stride;
     const float *   add;       // optional residual, column c at add + c * add_stride
@@ -130,8 +160,8 @@ struct gemm_launch {
 
 bool gemm_supported(int type, int64_t K, int64_t n_rows);
 void launch_gemm(const gemm_launch & G, hipStream_t st);
-// the workgroup tile launch_gemm picks (kernel template arguments: "4x4x2", "2x4x2", "1x2x4" for
-// Q4_0 / Q8_0 warp tiles x k-blocks; "2x2", "1x2" for the K-quants), for profile names
+// the workgroup tile launch_gemm picks (kernel template arguments: "4x4x2", "2x4x2", "1x2x4": wave
+// tiles x k-blocks), for profile names
 const char * gemm_tile_name(const gemm_launch & G);
 
 // Activation prologue of a GEMV: every workgroup quantizes its column of x itself, either as
@@ -172,8 +202,8 @@ struct gemv_launch {
     int        ncols;
     int        n_mats;
     gemv_mat   m[GEMV_MAX_MATS];
-    // activation (already quantized; column c at +c*K int8 and +c*K/32 (q8) or K/256 (q8K) scales),
-    // unused when norm.x is set
+    // activation (already quantized; column c at +c*K int8 and +c*K/32 (q8) or K/256 (q8K) scales;
+    // launch_mm_kq: xq is the x16 form), unused when norm.x is set
     const int8_t *  xq;
     const float *   xd;
     const int32_t * xs;    // q8: block sums
@@ -215,10 +245,6 @@ void launch_gemv_q(const gemv_launch & L, hipStream_t st);
 bool gemv_q4k_enabled();
 bool gemv_q4k_supported(const gemv_launch & L);
 void launch_gemv_q4k(const gemv_launch & L, hipStream_t st);
-// Dense Q4_K products of 2 or more pre-quantized columns with K <= 4096 on the matrix cores
-// (k_gemv_mfma.hip): 16 rows x 16 columns per workgroup, the same floats as the GEMV
-bool gemv_mfma_supported(const gemv_launch & L);
-void launch_gemv_mfma(const gemv_launch & L, hipStream_t st);
 // Several activation columns per workgroup (k_gemv_mc.hip): each weight row block is read once for
 // up to GEMV_MC_MAX_COLS columns; the activation must be quantized already (L.xq, no L.norm). With
 // groups (mul_mat_id): the workgroups of expert e take the columns the ids route to e, listed by
@@ -239,6 +265,23 @@ bool gemv_mc_fits(int type, int K, bool swiglu, int nc = 0);
 void launch_gemv_mc(const gemv_launch & L, const expert_groups * G, int max_cols, hipStream_t st);
 void launch_moe_group(const int32_t * ids, int64_t ids_stride, int n_slots, int n_tok, int n_experts, const expert_groups & g,
                       hipStream_t st);
+// Products of 2 or more Q8_K columns (x16 form, L.xq) with K-quant weights on the matrix cores
+// (k_mm_kq.hip): dense, or a mul_mat_id's columns grouped by expert (G). The same floats as the GEMV.
+enum mm_shape { MM_64x64, MM_64x48, MM_32x64, MM_64x32, MM_64x16, MM_16x16, MM_SPLIT, MM_RES2, MM_RES4, MM_RES8, MM_RES16 };
+constexpr size_t MM_RES_MAX_LDS = 78 * 1024;      // two workgroups per CU
+constexpr size_t mm_res_lds(int K, int nc) { return (size_t) (K / 256) * X16_USED * (nc <= 2 ? 2 : nc <= 4 ? 4 : nc <= 8 ? 8 : 16) * 16; }
+mm_shape mm_shape_of(const gemv_launch & L, const expert_groups * G);
+const char * mm_shape_name(mm_shape s);
+void launch_mm_kq(const gemv_launch & L, const expert_groups * G, hipStream_t st);
+void mm_dispatch_q4_k(mm_shape s, const gemv_launch & L, const expert_groups * G, hipStream_t st);
+void mm_dispatch_q5_k(mm_shape s, const gemv_launch & L, const expert_groups * G, hipStream_t st);
+void mm_dispatch_q6_k(mm_shape s, const gemv_launch & L, const expert_groups * G, hipStream_t st);
+// most columns of a grouped mul_mat_id's item
+constexpr int MOE_GROUP_MAX_COLS = 32;
+void launch_mm_kq(const gemv_launch & L, const expert_groups * G, hipStream_t st);
+void mm_dispatch_q4_k(mm_shape s, const gemv_launch & L, const expert_groups * G, int lds_cols, hipStream_t st);
+void mm_dispatch_q5_k(mm_shape s, const gemv_launch & L, const expert_groups * G, int lds_cols, hipStream_t st);
+void mm_dispatch_q6_k(mm_shape s, const gemv_launch & L, const expert_groups * G, int lds_cols, hipStream_t st);
 // L.norm's prologue for L.ncols columns of L.K, written once to q8 (Q4_0/Q8_0 consumers) or q8k (Q4_K)
 void launch_act_quant(const gemv_launch & L, const q8_act & q8, const q8k_act & q8k, hipStream_t st);
 // consumers with more rows than this get the activation quantized once instead of per workgroup
@@ -313,8 +356,9 @@ constexpr int64_t ROPE_TABLE_MIN_TOKENS = 16;   // RoPE jobs over at least this 
 void launch_rope_table(const int32_t * pos, int64_t n_pos, const rope_params & p, const float * ff, float2 * out, hipStream_t st);
 
 void launch_soft_max(const tview & a, const tview * mask, const tview & dst, float scale, float max_bias, hipStream_t st);
-// dst = silu(gate) * up (2-D f32 views), with its Q8_0 (q) or Q8_K (qk) quantization when set
-void launch_swiglu(const tview & gate, const tview & up, const tview & dst, const q8_act * q, const q8k_act * qk, hipStream_t st);
+// dst = silu(gate) * up (2-D f32 views), with its Q8_0 (q) or Q8_K (qk) quantization when set; without
+// keep only that quantization may be written
+void launch_swiglu(const tview & gate, const tview & up, const tview & dst, const q8_act * q, const q8k_act * qk, bool keep, hipStream_t st);
 
 // ---------------------------------------------------------------------------------------------
 // MoE routing and expert combination

@@ -25,7 +25,7 @@ GGML_API ggml_backend_buffer_type_t ggml_backend_hip_buffer_type(int device);
 // ---- extensions of this backend (no counterpart in the reference) ----
 
 // Bytes of device scratch ggml_backend_hip_graph_compute_static can give a graph's kernels.
-#define GGML_HIP_STATIC_SCRATCH_BYTES (64 << 20)
+#define GGML_HIP_STATIC_SCRATCH_BYTES (136 << 20)
 
 // ggml_backend_graph_compute without any device allocation: no counterpart in the reference; for
 // callers that cannot allocate (serving loops, harnesses that forbid hipMalloc). The kernels'

@@ -1,0 +1,79 @@
+"""Products of several activation columns at the edges of their workgroup shapes (rows and columns
+that end inside a tile, one super-block, several chunks), dense and routed, against the oracle: the
+same floats (every kernel adds the oracle's terms in the oracle's order)."""
+import numpy as np
+import pytest
+
+from gl import cpu_backend, gl, moe_ffn_graph, quantize, rel_err, run_on
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+    b = gl.hip_backend(0)
+    yield b
+    gl.libs()["core"].ggml_backend_free(b)
+
+
+@pytest.fixture(scope="module")
+def cpu():
+    b = cpu_backend(16)
+    yield b
+    gl.libs()["core"].ggml_backend_free(b)
+
+
+def rng(seed):
+    return np.random.default_rng(seed)
+
+
+def qweight(qtype, K, N, seed, std=0.02):
+    return quantize((rng(seed).standard_normal((N, K)) * std).astype(np.float32), qtype, impl="product")
+
+
+KQUANTS = [gl.Q4_K, gl.Q5_K, gl.Q6_K]
+
+
+@pytest.mark.parametrize("qtype", KQUANTS)
+@pytest.mark.parametrize("K,N,ncols", [
+    (256, 16420, 17),    # a 64-row workgroup per CU, the second column tile with one column
+    (256, 9000, 2),      # one-wave workgroups
+    (4352, 100, 33),     # K over eight waves: three chunks, the last with one super-block
+    (512, 4112, 250),    # 64 x 48 tiles, rows and columns ending inside one
+    (768, 530, 65),      # 32 x 64 tiles
+])
+def test_kquant_columns(hip, cpu, qtype, K, N, ncols):
+    w = qweight(qtype, K, N, K + N)
+    x = rng(ncols).standard_normal((ncols, K)).astype(np.float32)
+    x[0] = 0.0                      # a column of zero super-blocks
+    x[1, :256] = 1.5                # one whose values are all the largest
+    x[1, ::3] *= -1.0
+
+    def build(g):
+        return g.mul_mat(g.tensor(qtype, K, N, data=w), g.tensor(gl.F32, K, ncols, data=x))
+
+    a, b = run_on(hip, build), run_on(cpu, build)
+    assert np.array_equal(a, b), rel_err(a, b)
+
+
+@pytest.mark.parametrize("qtype", KQUANTS)
+@pytest.mark.parametrize("n_embd,ff,E,k,n_tok", [
+    (512, 256, 8, 4, 130),     # items of up to 32 columns
+    (2304, 256, 16, 4, 40),    # items of 16 columns whose K does not fit the LDS at once
+    (512, 512, 16, 2, 33),     # items of 8
+    (256, 256, 64, 8, 4),      # items of 2, most experts without a column
+])
+def test_kquant_expert_columns(hip, cpu, qtype, n_embd, ff, E, k, n_tok):
+    r = rng(n_embd + n_tok)
+    y, res = (r.standard_normal((n_tok, n_embd)).astype(np.float32) for _ in range(2))
+    router = (r.standard_normal((E, n_embd)) * 0.05).astype(np.float32)
+    wg, wu = (qweight(qtype, n_embd, E * ff, s, std=0.05) for s in (71, 72))
+    wd = qweight(qtype, ff, E * n_embd, 73, std=0.05)
+
+    def build(g):
+        return moe_ffn_graph(g, g.tensor(gl.F32, n_embd, n_tok, data=y), g.tensor(gl.F32, n_embd, E, data=router),
+                             g.tensor(qtype, n_embd, ff, E, data=wg), g.tensor(qtype, n_embd, ff, E, data=wu),
+                             g.tensor(qtype, ff, n_embd, E, data=wd), k, g.tensor(gl.F32, n_embd, n_tok, data=res))
+
+    a, b = run_on(hip, build), run_on(cpu, build)
+    assert np.array_equal(a, b), rel_err(a, b)
