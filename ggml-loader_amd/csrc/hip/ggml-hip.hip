@@ -1924,10 +1924,11 @@ private:
         return true;
     }
 
-    // the prefill attention kernel: a row of scores fits its LDS, K and V rows 16-byte aligned
-    static bool prefill_attn_ok(int64_t n_kv, int64_t hd, const void * k, size_t k_nb_a, size_t k_nb_b,
-                                const void * v, size_t v_nb_a, size_t v_nb_b) {
-        return n_kv <= attn_prefill_max_kv((int) hd) && ((uintptr_t) k | (uintptr_t) v) % 16 == 0 &&
+    // the prefill attention kernel: n_kv in its range for this many queries, K and V rows 16-byte aligned
+    static bool prefill_attn_ok(int64_t n_kv, int64_t n_q, int64_t n_head, int64_t n_head_kv, int64_t hd,
+                                const void * k, size_t k_nb_a, size_t k_nb_b, const void * v, size_t v_nb_a, size_t v_nb_b) {
+        return (n_kv <= attn_prefill_max_kv((int) hd) ||
+                attn_prefill_long_ok((int) n_kv, (int) n_q, (int) n_head, (int) n_head_kv)) && ((uintptr_t) k | (uintptr_t) v) % 16 == 0 &&
                k_nb_a % 16 == 0 && k_nb_b % 16 == 0 && v_nb_a % 16 == 0 && v_nb_b % 16 == 0;
     }
 
@@ -1970,7 +1971,7 @@ private:
         if (kp->nb[0] != 2 || vp->nb[1] != 2 || qp->nb[0] != 4) return false;
         if (n_q < 1 || n_head % n_head_kv) return false;
         if (hd != 64 && hd != 96 && hd != 128) return false;
-        if (n_q > 4 && !prefill_attn_ok(n_kv, hd, kp->data, kp->nb[1], kp->nb[2], vp->data, vp->nb[0], vp->nb[2]) &&
+        if (n_q > 4 && !prefill_attn_ok(n_kv, n_q, n_head, n_head_kv, hd, kp->data, kp->nb[1], kp->nb[2], vp->data, vp->nb[0], vp->nb[2]) &&
             n_head / n_head_kv > 8) return false;
         if (n_q <= 4 && n_head / n_head_kv > 8) return false;
         if (ctn->ne[0] != hd * n_head || ctn->ne[1] != n_q) return false;
@@ -1984,8 +1985,23 @@ private:
         return true;
     }
 
+    // score rows of the prefill attention that do not stay in registers: one buffer for the graph's
+    // launches, which the stream runs one after another
+    void prefill_scratch(attn_launch & A) {
+        A.scratch_bytes = attn_prefill_scratch_bytes(A.n_kv, A.n_q, A.n_head, A.n_head_kv, c_.scratch.fixed);
+        A.scratch = nullptr;
+        if (!A.scratch_bytes) return;
+        if (A.scratch_bytes > prefill_bytes_) {
+            prefill_buf_ = (float *) c_.scratch.alloc((size_t) A.scratch_bytes);
+            prefill_bytes_ = A.scratch_bytes;
+        }
+        A.scratch = prefill_buf_;
+    }
+    float * prefill_buf_ = nullptr;
+    int64_t prefill_bytes_ = 0;
+
     // More queries than the fused decode path takes, over more positions than the prefill kernel
-    // holds in LDS (a multi-token step deep into the context): the decode kernels, whose workgroups
+    // takes for so few (a multi-token step deep into the context): the decode kernels, whose workgroups
     // take 4 queries each, over up to ATT_DECODE_MAX_Q queries per launch, each launch with its own
     // rows of Q, mask and output (same arithmetic per query).
     void attn_decode_grouped(const attn_launch & A0) {
@@ -2087,7 +2103,8 @@ private:
         }
         const double bytes = (double) n_kv * n_head_kv * hd * 2 * 2 + (double) n_head * hd * n_q * 8 +
                              (mask ? (double) n_kv * n_q * ggml_type_size(mask->type) : 0.0);
-        if (n_q > 4 && prefill_attn_ok(n_kv, hd, kp->data, kp->nb[1], kp->nb[2], vp->data, vp->nb[0], vp->nb[2])) {
+        if (n_q > 4 && prefill_attn_ok(n_kv, n_q, n_head, n_head_kv, hd, kp->data, kp->nb[1], kp->nb[2], vp->data, vp->nb[0], vp->nb[2])) {
+            prefill_scratch(A);
             prof_scope ps(this, "attn_prefill", bytes);
             launch_attn_prefill(A, st_);
         } else if (n_q > 4) {
@@ -2122,7 +2139,7 @@ private:
                         q->type == GGML_TYPE_F32 && q->nb[0] == 4 && k->nb[0] == 2 && v->nb[0] == 2 && v->ne[0] == hd &&
                         n_q >= 1 && n_head % n_head_kv == 0 &&
                         (n_head / n_head_kv <= 8 ||
-                         (n_q > 4 && prefill_attn_ok(n_kv, hd, k->data, k->nb[1], k->nb[2], v->data, v->nb[1], v->nb[2]))) &&
+                         (n_q > 4 && prefill_attn_ok(n_kv, n_q, n_head, n_head_kv, hd, k->data, k->nb[1], k->nb[2], v->data, v->nb[1], v->nb[2]))) &&
                         (hd == 64 || hd == 96 || hd == 128) && ggml_is_contiguous(n) &&
                         ((uintptr_t) k->data) % 16 == 0 && k->nb[1] % 16 == 0 && k->nb[2] % 16 == 0 &&
                         ((uintptr_t) v->data) % 4 == 0 && v->nb[1] % 4 == 0 && v->nb[2] % 4 == 0 &&
@@ -2148,7 +2165,8 @@ private:
         A.skip_masked = 1;
         A.p_f32 = 1;
         const double bytes = (double) n_kv * n_head_kv * hd * 2 * 2 + (double) n_head * hd * n_q * 8;
-        if (n_q > 4 && prefill_attn_ok(n_kv, hd, k->data, k->nb[1], k->nb[2], v->data, v->nb[1], v->nb[2])) {
+        if (n_q > 4 && prefill_attn_ok(n_kv, n_q, n_head, n_head_kv, hd, k->data, k->nb[1], k->nb[2], v->data, v->nb[1], v->nb[2])) {
+            prefill_scratch(A);
             prof_scope ps(this, "attn_prefill", bytes);
             launch_attn_prefill(A, st_);
             return;

@@ -817,6 +817,8 @@ __global__ __launch_bounds__(ATT_THREADS) void attn_pv_kernel(const attn_launch 
 // f64 MFMA 16x16x4 lane layout: A[i][k] at lane i + 16k, B[k][j] at lane j + 16k, D[i][j] in
 // register i / 4 of lane j + 16 (i % 4).
 typedef double v4d __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4a __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int MQ_ROWS = 16;
 
@@ -1260,376 +1262,382 @@ void launch_attn_decode(const attn_launch & A_in, hipStream_t st) {
 
 // ---------------------------------------------------------------------------------------------
 // Prefill attention: the same chain arithmetic for a batch of queries (n_q > 4), one workgroup per
-// (tile of APF_Q queries, head), all of a row's scores held in LDS.
-//   scores  K rows staged per 64-position chunk; S[query][pos] from v_mfma_f64_16x16x4f64 over the
-//           head dimension (the F16 operands are exact in double, the sum accumulates in double as
-//           the chain's), rounded to float, times scale, plus mask. A chunk whose mask is -inf for
-//           every query of the tile is not computed: its scores are -inf, as the chain forms them.
+// (KV head, tile of 16 of its (query, head) rows). Wave w takes the 16-position tiles w, w + WAVES, ...
+//   mask    the tile's mask, for the tiles that no row sees: those are not computed (their scores are
+//           -inf, as the chain forms them, and their p are 0).
+//   scores  S^T[position][row] from v_mfma_f64_16x16x4f64 over the head dimension (the F16 operands
+//           are exact in double, the sum accumulates in double as the chain's), rounded to float,
+//           times scale, plus mask. The sum over the head dims is exact in any order, so lane group
+//           g = lane / 16 takes the NJ consecutive dims NJ g .. (MFMA step j: dim NJ g + j) and a
+//           lane's K operands are 16-byte pieces of its position's row, loaded straight into registers.
 //   stats   per row: M = max, e = exp(s - M), S = sum e in double, p = F16(e * (float)(1/S))
-//           (flash_attn_ext, p_f32: p = e * (float)(1/S), not rounded to F16).
-//   pv      V rows staged per chunk; out[query][dim] from the f64 MFMA over positions with the
-//           p (skipped chunks have p = 0 throughout and add nothing), rounded to float.
+//           (flash_attn_ext, p_f32: p = e * (float)(1/S), not rounded to F16). A lane holds scores of
+//           one row only, so these are sums over its own scores, then over 4 lanes and the waves.
+//   pv      out^T[dim][row] += V^T P^T: score r of a lane is its B operand of MFMA step r (positions
+//           4 r .. 4 r + 3) as it stands. Output tile k, row i is dim i NT + k, so that the A operands
+//           of all NT tiles are NT consecutive halves of a V row: one load per step. The waves'
+//           partial sums are added in LDS (double sums, exact in practice).
+// A lane keeps its scores (4 per tile) in registers, PT tiles at most, or (PT = 0) in its own 16 bytes
+// per tile of a scratch buffer that only it reads again: no LDS in the loops, no barrier but between
+// the phases. The f64 pipe bounds it: the f64 matrix instructions (2 n_q n_kv hd multiply-adds per head,
+// 29 ns per 16x16x4 and SIMD, 72 TFLOP/s) and the vector instructions of every wave of a SIMD take turns
+// (measured: 8 vector instructions between two of them add their whole 16 ns), so what counts beside them
+// is the number of vector instructions: K and V converted F16 -> F32 -> F64, the exps in double. Two row
+// tiles per workgroup (K and V converted once for both) gained 3% at 1000 queries over 4001 positions
+// and lost 9 to 20% where the doubled workgroups fill the CUs badly (300 over 1800, 640 over 8832).
+// Measured (us a launch; before: score rows in LDS up to 2176 positions at head dim 128, K and V through
+// LDS; past it the multi-query kernels above in groups of 64 queries): Phi-3 heads (32 x 96), 512 queries over
+// 512 positions 81 -> 66; GQA (32 heads, 8 KV, 128), 1000 over 4001 2240 -> 1480 (39 TFLOP/s).
 // (f64 MFMA lane layout as above.)
-constexpr int APF_Q = 16;           // queries per workgroup (one MFMA row tile)
-constexpr int APF_CHUNK = 64;        // positions per staged K / V chunk (one MFMA column tile per wave)
-constexpr int APF_MAX_CHUNKS = 128;  // positions <= 8192
+constexpr int APF_ROWS = 16;           // (query, head) rows per workgroup
+constexpr int APF_MAX_TILES = 4096;    // positions <= 65536
+constexpr int APF_REG_KV = 16 * 32 * 8;  // positions whose scores a CU's registers hold
+constexpr int APF_CUS = 256;             // compute units
+constexpr int APF_MAX_BLOCKS = 512;      // workgroups with scores in scratch
 
-template <int HD>
-constexpr int apf_static_lds() {
-    return (APF_Q + APF_CHUNK) * (HD + 2) * 2 + APF_MAX_CHUNKS * 4;
-}
+template <int PT> struct score_vec { typedef float t __attribute__((ext_vector_type(PT))); };
+template <> struct score_vec<0> { typedef float t __attribute__((ext_vector_type(2))); };   // not used
 
-__host__ __device__ inline int apf_row_stride(int n_kv) {
-    return (n_kv + APF_CHUNK - 1) / APF_CHUNK * APF_CHUNK + 4;   // floats; +4 spreads rows over banks
-}
-
-template <int HD>
-__global__ __launch_bounds__(ATT_THREADS) void attn_prefill_kernel(const attn_launch A) {
+template <int HD, int PT, int WAVES, bool FLASH>
+__global__ __launch_bounds__(64 * WAVES, PT == 8 ? 3 : 2) void attn_prefill_kernel(const attn_launch A) {
     prefetch_kernargs<sizeof(attn_launch)>();
-    constexpr int KSTR = HD + 2;     // halves per staged row (one dword of padding)
-    constexpr int PIECES = HD / 8;   // 16-byte pieces per row
-    __shared__ __half s_q[APF_Q * KSTR];
-    __shared__ __half s_kv[APF_CHUNK * KSTR];
-    __shared__ int s_live[APF_MAX_CHUNKS];
-    __shared__ int s_live_end;       // one past the last live chunk
-    extern __shared__ float s_s[];   // [APF_Q][SS]: scores, then e, then p
-    // the last query tiles first, every head's before any head's shorter ones (the head is the
-    // fastest grid index): under a causal mask they see the most positions, and started last they
-    // would leave the chip waiting on a few long workgroups
-    const int q0 = (gridDim.y - 1 - blockIdx.y) * APF_Q, h = blockIdx.x;
-    const int kvh = h / (A.n_head / A.n_head_kv);
-    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-    const int n_kv = A.n_kv, n_q = A.n_q;
-    const int SS = apf_row_stride(n_kv);
-    const int n_chunks = (n_kv + APF_CHUNK - 1) / APF_CHUNK;
-    const __half * kbase = A.k + (int64_t) kvh * A.k_nb1;
-    const __half * vbase = A.v + (int64_t) kvh * A.v_nb1;
+    constexpr int NJ = HD / 4, KU = NJ / 8;      // dims per lane group, 16-byte pieces of a lane's K slice
+    constexpr int NT = HD / 16;                  // output tiles: halves of a lane's V piece
+    static_assert(NJ % 8 == 0 && NT % 2 == 0, "whole 16-byte K pieces, whole dwords of V");
+    constexpr int MB = PT ? 8 : 2;               // tiles per batch of mask loads
+    constexpr int MAXP = PT ? PT : (APF_MAX_TILES + WAVES - 1) / WAVES;
+    constexpr bool QLDS = PT == 0 || PT == 32;
+    __shared__ __align__(16) double2 s_q[QLDS ? NJ / 2 : 1][WAVE];
+    __shared__ float s_m[WAVES][APF_ROWS];
+    __shared__ double s_s[WAVES][APF_ROWS];
+    __shared__ uint16_t s_dead[WAVES][MAXP];     // per tile of a wave, bit 4 g + r: no row sees position g + 4 r
+    __shared__ __align__(16) double s_red[WAVES / 2][APF_ROWS * HD];
+    const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x / WAVE);
+    const int c = lane % 16, g = lane / 16;
+    const int G = A.n_head / A.n_head_kv, n_rows = A.n_q * G, n_kv = A.n_kv;
+    const int n_tiles = (n_kv + 15) / 16, my = (n_tiles - wave + WAVES - 1) / WAVES;   // tiles, this wave's
+    f32x4 * own = PT ? nullptr : (f32x4 *) A.scratch + ((int64_t) blockIdx.x * n_tiles + wave) * WAVE + lane;   // tile p at own[p WAVES 64]
+    // the KV head is the fastest grid index (a head's workgroups then share an XCD's L2 where the
+    // heads are a multiple of the XCDs); the last row tiles, the longest under a causal mask, first.
+    // With the scores in scratch a workgroup takes several row tiles, one after another.
+    const int n_row_tiles = (n_rows + APF_ROWS - 1) / APF_ROWS;
+    int item = blockIdx.x;
+    do {
+    const int kvh = item % A.n_head_kv, r0 = (n_row_tiles - 1 - item / A.n_head_kv) * APF_ROWS;
+    const int row = min(r0 + c, n_rows - 1);     // rows past the end repeat the last one; not stored
+    const int q = row / G, h = kvh * G + row % G;
 
-    // Q tile rounded to F16 (rows past n_q repeat the last query; their results are not stored)
-    for (int i = threadIdx.x; i < APF_Q * HD; i += ATT_THREADS) {
-        const int qi = i / HD, d = i % HD;
-        const int q = min(q0 + qi, n_q - 1);
-        s_q[qi * KSTR + d] = __float2half_rn(A.q[(int64_t) h * A.q_nb1 + (int64_t) q * A.q_nb2 + d]);
-    }
-
-    // rows [t0, t0 + nt) of a cache view into registers, and from there into s_kv (zero past nt;
-    // with zero_dead, rows masked for every query of the tile also read as zero: skip_masked). The
-    // loads are unconditional, at clamped rows, and the zeroing happens at the LDS store: a guarded
-    // load, or a register zeroed right after its load, makes the compiler wait for every load.
-    static_assert(APF_CHUNK * PIECES % ATT_THREADS == 0, "whole 16-byte pieces per thread");
-    constexpr int ITER = APF_CHUNK * PIECES / ATT_THREADS;
-    auto load_rows = [&](uint4 (&v)[ITER], const __half * base, int64_t nb_pos, int t0, int nt) {
-#pragma unroll
-        for (int it = 0; it < ITER; it++) {
-            const int pc = threadIdx.x + it * ATT_THREADS;
-            const int r = pc / PIECES, c = pc % PIECES;
-            v[it] = *(const uint4 *) (base + (int64_t) (t0 + min(r, nt - 1)) * nb_pos + c * 8);
-        }
-    };
-    auto store_rows = [&](uint4 (&v)[ITER], int t0, int nt, bool zero_dead) {
-        bool zero[ITER];
-#pragma unroll
-        for (int it = 0; it < ITER; it++) zero[it] = (threadIdx.x + it * ATT_THREADS) / PIECES >= nt;
-        if (zero_dead) {
-#pragma unroll
-            for (int it = 0; it < ITER; it++) {
-                const int r = (threadIdx.x + it * ATT_THREADS) / PIECES;
-                bool dead = r < nt;
-                for (int q = q0; q < min(q0 + APF_Q, n_q) && dead; q++) dead = mask_at(A, q, t0 + r) == -INFINITY;
-                zero[it] = zero[it] || dead;
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < ITER; it++) {
-            const int pc = threadIdx.x + it * ATT_THREADS;
-            const int r = pc / PIECES, c = pc % PIECES;
-            uint32_t * d = (uint32_t *) (s_kv + r * KSTR + c * 8);
-            const bool z = zero[it];
-            d[0] = z ? 0u : v[it].x; d[1] = z ? 0u : v[it].y; d[2] = z ? 0u : v[it].z; d[3] = z ? 0u : v[it].w;
-        }
-    };
-    auto next_live = [&](int ch) {
-        while (ch < n_chunks && !s_live[ch]) ch++;
-        return ch;
-    };
-
-    // the tile's mask rows into s_s (rows past n_q repeat the last query's; 0 without a mask), read
-    // once here instead of in every chunk: one position per thread and row at a time, the loads of
-    // all APF_Q rows in flight together (unconditional, at clamped positions)
-    if (threadIdx.x == 0) s_live_end = 0;
-    auto stage_mask = [&](auto load) {
-        for (int t0 = 0; t0 < n_kv; t0 += ATT_THREADS) {
-            const int t = min(t0 + (int) threadIdx.x, n_kv - 1);
-            float v[APF_Q];
-#pragma unroll
-            for (int qi = 0; qi < APF_Q; qi++) v[qi] = load(min(q0 + qi, n_q - 1), t);
-            if (t0 + (int) threadIdx.x < n_kv) {
-#pragma unroll
-                for (int qi = 0; qi < APF_Q; qi++) s_s[qi * SS + t] = v[qi];
-            }
-        }
-    };
-    if (!A.mask) {
-        stage_mask([&](int, int) { return 0.0f; });
-    } else if (A.mask_f16 && n_kv % 8 == 0 && A.mask_nb1 % 16 == 0 && (uintptr_t) A.mask % 16 == 0) {
-        // eight positions per 16-byte load, up to eight loads in flight per thread
-        const int per_row = n_kv / 8, total = APF_Q * per_row;
-        for (int base = 0; base < total; base += 8 * ATT_THREADS) {
-            uint4 v[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int i = min(base + u * ATT_THREADS + (int) threadIdx.x, total - 1);
-                const int qi = i / per_row, pc = i % per_row;
-                v[u] = *(const uint4 *) ((const char *) A.mask + (int64_t) min(q0 + qi, n_q - 1) * A.mask_nb1 + pc * 16);
-            }
-#pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int i = base + u * ATT_THREADS + (int) threadIdx.x;
-                if (i < total) {
-                    const int qi = i / per_row, pc = i % per_row;
-                    const uint32_t w[4] = { v[u].x, v[u].y, v[u].z, v[u].w };
-                    float f[8];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const float2 x2 = __half22float2(*(const __half2 *) &w[e]);
-                        f[2 * e] = x2.x;
-                        f[2 * e + 1] = x2.y;
-                    }
-                    float4 * d = (float4 *) (s_s + qi * SS + pc * 8);
-                    d[0] = make_float4(f[0], f[1], f[2], f[3]);
-                    d[1] = make_float4(f[4], f[5], f[6], f[7]);
-                }
-            }
-        }
-    } else if (A.mask_f16) {
-        stage_mask([&](int q, int t) { return __half2float(((const __half *) ((const char *) A.mask + (int64_t) q * A.mask_nb1))[t]); });
-    } else {
-        stage_mask([&](int q, int t) { return ((const float *) ((const char *) A.mask + (int64_t) q * A.mask_nb1))[t]; });
-    }
-    __syncthreads();
-    // chunk liveness, one wave per chunk (lane = position): a chunk whose mask is -inf for every
-    // query of the tile is not computed. Its staged values are then -inf in every row (rows past
-    // n_q repeat the last query's), which are the scores the chain forms for it.
-    static_assert(APF_CHUNK == WAVE, "one position per lane");
-    for (int ch = wave; ch < n_chunks; ch += ATT_WAVES) {
-        const int t = ch * APF_CHUNK + lane;
-        bool any = !A.mask;
-        if (t < n_kv) {
-            float v[APF_Q];
-#pragma unroll
-            for (int qi = 0; qi < APF_Q; qi++) v[qi] = s_s[qi * SS + t];
-#pragma unroll
-            for (int qi = 0; qi < APF_Q; qi++) any = any || (q0 + qi < n_q && v[qi] != -INFINITY);
-        }
-        const bool live = __any(any);
-        if (lane == 0) {
-            s_live[ch] = live;
-            if (live) atomicMax(&s_live_end, ch + 1);
-        }
-    }
-    __syncthreads();
-
-    // ---- scores, over the live chunks; wave w takes positions 16 w .. 16 w + 15 of each. The sum
-    // over the head dims is exact in any order, so lane group g = lane / 16 takes the NJ consecutive
-    // dims NJ g .. NJ g + NJ - 1 (MFMA step j: dim NJ g + j): a lane's K operands are NJ / 8
-    // 16-byte pieces of its position's row, loaded straight into registers (no LDS, no barrier),
-    // the next live chunk's while this one is used. Q as the A operands, converted once: lane
-    // (i + 16 g) holds Q[i][NJ g + j]. ----
-    constexpr int NJ = HD / 4;
-    constexpr int KU = NJ / 8;                   // 16-byte pieces of a lane's K slice
-    static_assert(NJ % 8 == 0, "whole 16-byte K pieces per lane");
-    double qd[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; j++) qd[j] = (double) __half2float(s_q[(lane % 16) * KSTR + NJ * (lane / 16) + j]);
-    const __half * kslice = kbase + NJ * (lane / 16);
-    auto load_k = [&](uint4 (&v)[KU], int c) {
-        const int t = min(c * APF_CHUNK + wave * 16 + lane % 16, n_kv - 1);   // clamped, unused past the end
-        const uint4 * src = (const uint4 *) (kslice + (int64_t) t * A.k_nb2);
-#pragma unroll
-        for (int u = 0; u < KU; u++) v[u] = src[u];
-    };
-    uint4 kc[KU], kn[KU];
-    int ch = next_live(0);
-    if (ch < n_chunks) load_k(kc, ch);
-    while (ch < n_chunks) {
-        const int t0 = ch * APF_CHUNK, nt = min(APF_CHUNK, n_kv - t0);
-        const int nx = next_live(ch + 1);
-        if (nx < n_chunks) load_k(kn, nx);
-        // two independent accumulation chains (even and odd steps), added at the end: the double
-        // sums are exact for these operands, so the grouping does not matter
-        v4d acc = { 0.0, 0.0, 0.0, 0.0 }, acc2 = { 0.0, 0.0, 0.0, 0.0 };
-        uint32_t kw[NJ / 2];
-        __builtin_memcpy(kw, kc, sizeof(kw));
+    // this lane's slice of its Q row, rounded to F16 (the mul_mat's conversion of its F32 operand), as
+    // doubles: in registers, or where those are short in LDS (every wave stores the same and reads its own lane's)
+    double qd[QLDS ? 1 : NJ];
+    {
+        const float * src = A.q + (int64_t) h * A.q_nb1 + (int64_t) q * A.q_nb2 + NJ * g;
 #pragma unroll
         for (int j = 0; j < NJ; j += 2) {
-            const float2 b = __half22float2(*(const __half2 *) &kw[j / 2]);
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(qd[j], (double) b.x, acc, 0, 0, 0);
-            acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(qd[j + 1], (double) b.y, acc2, 0, 0, 0);
+            const double2 v = make_double2((double) __half2float(__float2half_rn(src[j])), (double) __half2float(__float2half_rn(src[j + 1])));
+            if constexpr (QLDS) s_q[j / 2][lane] = v;
+            else { qd[j] = v.x; qd[j + 1] = v.y; }
         }
-        acc += acc2;
-        const int t = wave * 16 + lane % 16;
-        if (t < nt) {
+    }
+    // the mask of this lane's row at positions g + 4 r of NP tiles from the wave's tile p (-inf past the end)
+    const char * mrow = (const char *) A.mask + (int64_t) q * A.mask_nb1;
+    auto load_mask = [&](auto & m, int p, auto np) {
+        constexpr int NP = decltype(np)::value;
+        auto at = [&](int i, int r) { return min(16 * (wave + WAVES * (p + i)) + g + 4 * r, n_kv - 1); };
+        if (!A.mask) {
+#pragma unroll
+            for (int i = 0; i < NP; i++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) m[i][r] = 0.0f;
+        } else if (A.mask_f16) {
+            __half v[NP][4];
+#pragma unroll
+            for (int i = 0; i < NP; i++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[i][r] = ((const __half *) mrow)[at(i, r)];
+#pragma unroll
+            for (int i = 0; i < NP; i++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) m[i][r] = __half2float(v[i][r]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NP; i++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) m[i][r] = ((const float *) mrow)[at(i, r)];
+        }
+#pragma unroll
+        for (int i = 0; i < NP; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (16 * (wave + WAVES * (p + i)) + g + 4 * r >= n_kv) m[i][r] = -INFINITY;
+    };
+
+    // ---- mask: the dead positions of every tile; the mask itself kept where the scores will be ----
+    typename score_vec<PT>::t sc[4];             // sc[r][p]: position 16 (wave + WAVES p) + g + 4 r
+    auto dead_of = [&](const float (&m)[4]) {
+        uint32_t d = 0;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const uint64_t b = __ballot(m[r] != -INFINITY);
+#pragma unroll
+            for (int gg = 0; gg < 4; gg++) if (((b >> (16 * gg)) & 0xffff) == 0) d |= 1u << (4 * gg + r);
+        }
+        return d;
+    };
+    // (every lane stores the same value and reads it again itself)
+#pragma unroll
+    for (int p = 0; p < (PT ? PT : my); p += MB) {
+        float m[MB][4];
+        load_mask(m, p, std::integral_constant<int, MB>{});
+#pragma unroll
+        for (int i = 0; i < MB; i++) {
+            if (p + i < MAXP) s_dead[wave][p + i] = (uint16_t) dead_of(m[i]);
+            if constexpr (PT != 0) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) sc[r][p + i] = m[i][r];
+            }
+        }
+    }
+    auto dead_at = [&](int p) { return (uint32_t) __builtin_amdgcn_readfirstlane((int) s_dead[wave][p]); };
+    auto next_live = [&](int p) {
+        while (p < my && dead_at(p) == 0xffff) p++;
+        return p;
+    };
+
+    // ---- scores ----
+    struct tile_in { u32x4a k[KU]; float m[1][4]; };
+    const __half * kslice = A.k + (int64_t) kvh * A.k_nb1 + NJ * g;
+    auto load = [&](tile_in & T, int p) {
+        const u32x4a * src = (const u32x4a *) (kslice + (int64_t) min(16 * (wave + WAVES * p) + c, n_kv - 1) * A.k_nb2);
+#pragma unroll
+        for (int u = 0; u < KU; u++) T.k[u] = src[u];
+        if constexpr (PT == 0) load_mask(T.m, p, std::integral_constant<int, 1>{});
+    };
+    const int first = next_live(0);
+    float mx = -INFINITY;
+    {
+        tile_in cur, nxt;
+        int p = first;
+        if (p < my) load(cur, p);
+        while (p < my) {
+            const int np = next_live(p + 1);
+            load(nxt, np < my ? np : p);
+            v4d a0 = { 0.0, 0.0, 0.0, 0.0 }, a1 = { 0.0, 0.0, 0.0, 0.0 };
+#pragma unroll
+            for (int j = 0; j < NJ; j += 2) {
+                const uint32_t kw = cur.k[j / 8][j / 2 % 4];
+                const float2 kf = __half22float2(__builtin_bit_cast(__half2, kw));
+                const double2 qv = QLDS ? s_q[j / 2][lane] : make_double2(qd[QLDS ? 0 : j], qd[QLDS ? 0 : j + 1]);
+                a0 = __builtin_amdgcn_mfma_f64_16x16x4f64((double) kf.x, qv.x, a0, 0, 0, 0);
+                a1 = __builtin_amdgcn_mfma_f64_16x16x4f64((double) kf.y, qv.y, a1, 0, 0, 0);
+            }
+            f32x4 s;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int qi = lane / 16 + 4 * r;
-                float * sp = s_s + qi * SS + t0 + t;
-                const float mv = *sp;
-                *sp = mv == -INFINITY ? -INFINITY : (float) acc[r] * A.scale + mv;
+                const float mk = PT ? sc[r][p] : cur.m[0][r];
+                s[r] = mk == -INFINITY ? -INFINITY : (float) (a0[r] + a1[r]) * A.scale + mk;
+                mx = fmaxf(mx, s[r]);
+                if constexpr (PT != 0) sc[r][p] = s[r];
             }
+            if constexpr (PT == 0) own[(int64_t) p * (WAVES * WAVE)] = s;
+            cur = nxt;
+            p = np;
         }
-#pragma unroll
-        for (int u = 0; u < KU; u++) kc[u] = kn[u];
-        ch = nx;
     }
+    // ---- statistics ----
+    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+    if (g == 0) s_m[wave][c] = mx;
     __syncthreads();
-
-    // ---- row statistics and probabilities, over the positions before the end of the last live
-    // chunk (later ones are -inf, take no part in the sums and are never read again); unrolled so
-    // that independent exps interleave ----
-    const int n_pos = min(s_live_end * APF_CHUNK, n_kv);
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) mx = fmaxf(mx, s_m[w][c]);
+    const bool none = mx == -INFINITY;           // a row masked throughout gets e = 0
+    const float m0 = none ? 0.0f : mx;
+    double sum = 0.0;
     {
-        constexpr int RPW = APF_Q / ATT_WAVES;          // rows qi = wave + 4 k of this wave, together
-        float * row[RPW];
-        float m[RPW];
+        f32x4 cur, nxt;
+        int p = first;
+        if constexpr (PT == 0) if (p < my) cur = own[(int64_t) p * (WAVES * WAVE)];
+        while (p < my) {
+            const int np = next_live(p + 1);
+            if constexpr (PT == 0) nxt = own[(int64_t) (np < my ? np : p) * (WAVES * WAVE)];
+            f32x4 e;
 #pragma unroll
-        for (int k = 0; k < RPW; k++) {
-            row[k] = s_s + (wave + ATT_WAVES * k) * SS;
-            m[k] = -INFINITY;
-        }
-        for (int t = lane; t < n_pos; t += WAVE) {
-#pragma unroll
-            for (int k = 0; k < RPW; k++) m[k] = fmaxf(m[k], row[k][t]);
-        }
-#pragma unroll
-        for (int k = 0; k < RPW; k++) m[k] = wave_max(m[k]);
-        double sum[RPW];
-#pragma unroll
-        for (int k = 0; k < RPW; k++) sum[k] = 0.0;
-#pragma unroll 2
-        for (int t = lane; t < n_pos; t += WAVE) {
-#pragma unroll
-            for (int k = 0; k < RPW; k++) {
-                // a row masked throughout (m = -inf) gets p = 0
-                const float e = m[k] == -INFINITY ? 0.0f : exp_cr(row[k][t] - m[k]);
-                row[k][t] = e;
-                sum[k] += (double) e;
+            for (int r = 0; r < 4; r++) {
+                const float x = exp_cr((PT ? sc[r][p] : cur[r]) - m0);
+                e[r] = none ? 0.0f : x;
+                sum += (double) e[r];
+                if constexpr (PT != 0) sc[r][p] = e[r];
             }
-        }
-        float inv[RPW];
-#pragma unroll
-        for (int k = 0; k < RPW; k++) {
-            const double sk = wave_sum_d(sum[k]);
-            inv[k] = sk > 0.0 ? (float) (1.0 / sk) : 0.0f;
-        }
-        for (int t = lane; t < n_pos; t += WAVE) {
-#pragma unroll
-            for (int k = 0; k < RPW; k++) {
-                const float p = as_f32(row[k][t] * inv[k]);
-                row[k][t] = A.p_f32 ? p : __half2float(__float2half_rn(p));
+            if constexpr (PT == 0) {
+                own[(int64_t) p * (WAVES * WAVE)] = e;
+                cur = nxt;
             }
+            p = np;
         }
     }
+    sum += __shfl_xor(sum, 16, WAVE);
+    sum += __shfl_xor(sum, 32, WAVE);
+    if (g == 0) s_s[wave][c] = sum;
+    __syncthreads();
+    sum = s_s[0][c];
+#pragma unroll
+    for (int w = 1; w < WAVES; w++) sum += s_s[w][c];
+    const float inv = sum > 0.0 ? (float) (1.0 / sum) : 0.0f;
 
-    // ---- P V: wave w takes positions 16 w .. 16 w + 15 of every chunk for all HD / 16 output
-    // tiles; the four waves' partial sums are added at the end (double sums, exact in practice) ----
-    constexpr int NT = HD / 16;                  // 16-dim output tiles
+    // ---- P V ----
     v4d acc[NT];
 #pragma unroll
     for (int k = 0; k < NT; k++) acc[k] = v4d{ 0.0, 0.0, 0.0, 0.0 };
-    uint4 kv[ITER];
-    ch = next_live(0);
-    if (ch < n_chunks) load_rows(kv, vbase, A.v_nb2, ch * APF_CHUNK, min(APF_CHUNK, n_kv - ch * APF_CHUNK));
-    while (ch < n_chunks) {
-        const int t0 = ch * APF_CHUNK, nt = min(APF_CHUNK, n_kv - t0);
-        store_rows(kv, t0, nt, A.skip_masked && A.mask);
-        __syncthreads();                         // p of every row and this chunk's V rows visible
-        const int nx = next_live(ch + 1);
-        if (nx < n_chunks) load_rows(kv, vbase, A.v_nb2, nx * APF_CHUNK, min(APF_CHUNK, n_kv - nx * APF_CHUNK));
+    const __half * vcol = A.v + (int64_t) kvh * A.v_nb1 + NT * c;
+    struct vpiece { uint32_t w[NT / 2]; };       // NT consecutive halves of a V row
+    auto load_v = [&](vpiece & V, int p, int r) {
+        const int t = min(16 * (wave + WAVES * p) + 4 * r + g, n_kv - 1);
+        __builtin_memcpy(&V, vcol + (int64_t) t * A.v_nb2, sizeof(vpiece));
+    };
+    {
+        vpiece vc[4];                            // reloaded for the next tile as each is used up
+        f32x4 ecur, enxt;
+        int p = first;
+        if (p < my) {
 #pragma unroll
-        for (int s4 = 0; s4 < 4; s4++) {
-            const int t = 16 * wave + 4 * s4 + lane / 16;      // rows past nt are staged as zero
-            const double a = t < nt ? (double) s_s[(lane % 16) * SS + t0 + t] : 0.0;
-#pragma unroll
-            for (int k = 0; k < NT; k++) {
-                const double b = (double) __half2float(s_kv[t * KSTR + k * 16 + lane % 16]);
-                acc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[k], 0, 0, 0);
-            }
+            for (int r = 0; r < 4; r++) load_v(vc[r], p, r);
+            if constexpr (PT == 0) ecur = own[(int64_t) p * (WAVES * WAVE)];
         }
-        __syncthreads();                         // every wave's reads of this chunk's s_kv are done
-        ch = nx;
-    }
-    // register r of lane (c + 16 g) holds row g + 4 r, column c of each tile (the f64 MFMA's D
-    // layout); waves 2, 3 hand theirs to waves 0, 1, then wave 1 to wave 0 (the dynamic LDS holds
-    // 2 * APF_Q * HD doubles)
-    double * red = (double *) s_s;
-    auto red_at = [&](int slot, int k, int r) { return red + ((slot * APF_Q + lane / 16 + 4 * r) * HD + k * 16 + lane % 16); };
-    if (wave >= 2) {
-#pragma unroll
-        for (int k = 0; k < NT; k++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) *red_at(wave - 2, k, r) = acc[k][r];
-    }
-    __syncthreads();
-    if (wave < 2) {
-#pragma unroll
-        for (int k = 0; k < NT; k++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) acc[k][r] += *red_at(wave, k, r);
-    }
-    __syncthreads();
-    if (wave == 1) {
-#pragma unroll
-        for (int k = 0; k < NT; k++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) *red_at(0, k, r) = acc[k][r];
-    }
-    __syncthreads();
-    if (wave == 0) {
-#pragma unroll
-        for (int k = 0; k < NT; k++) {
+        while (p < my) {
+            const int after = next_live(p + 1), np = after < my ? after : p;
+            const bool tail = 16 * (wave + WAVES * p) + 16 > n_kv;
+            const uint32_t dead = FLASH ? dead_at(p) >> (4 * g) : 0;
+            if constexpr (PT == 0) enxt = own[(int64_t) np * (WAVES * WAVE)];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int q = q0 + lane / 16 + 4 * r;
-                const double v = acc[k][r] + *red_at(0, k, r);
-                if (q < n_q) A.out[(int64_t) q * A.out_nb1 + (int64_t) h * HD + k * 16 + lane % 16] = (float) v;
+                const float e = as_f32((PT ? sc[r][p] : ecur[r]) * inv);
+                const double b = (double) (FLASH ? e : __half2float(__float2half_rn(e)));
+                vpiece w = vc[r];
+                // V of a position past the end, or (flash_attn_ext) masked for every row, counts as
+                // zero: 0 * a non-finite V must not reach the sums
+                if ((FLASH && ((dead >> r) & 1)) || (tail && 16 * (wave + WAVES * p) + 4 * r + g >= n_kv)) {
+#pragma unroll
+                    for (int k = 0; k < NT / 2; k++) w.w[k] = 0u;
+                }
+#pragma unroll
+                for (int k = 0; k < NT; k += 2) {
+                    const float2 f = __half22float2(__builtin_bit_cast(__half2, w.w[k / 2]));
+                    acc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64((double) f.x, b, acc[k], 0, 0, 0);
+                    acc[k + 1] = __builtin_amdgcn_mfma_f64_16x16x4f64((double) f.y, b, acc[k + 1], 0, 0, 0);
+                }
+                load_v(vc[r], np, r);
+                __builtin_amdgcn_sched_barrier(0);
             }
+            if constexpr (PT == 0) ecur = enxt;
+            p = after;
         }
     }
-}
-
-static int max_lds_per_block() {
-    static int v = -1;
-    if (v < 0) {
-        int dev = 0;
-        HIP_CHECK(hipGetDevice(&dev));
-        HIP_CHECK(hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    // the upper half of the waves hands its sums to the lower half until one is left. Register r of
+    // lane (c, g): row c, dims (g + 4 r) NT + k
+#pragma unroll
+    for (int n = WAVES / 2; n >= 1; n /= 2) {
+        __syncthreads();
+        if (wave >= n && wave < 2 * n) {
+#pragma unroll
+            for (int k = 0; k < NT; k++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) s_red[wave - n][(k * 4 + r) * WAVE + lane] = acc[k][r];
+        }
+        __syncthreads();
+        if (wave < n) {
+#pragma unroll
+            for (int k = 0; k < NT; k++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[k][r] += s_red[wave][(k * 4 + r) * WAVE + lane];
+        }
     }
-    return v;
+    if (wave == 0 && r0 + c < n_rows) {
+        float * o = A.out + (int64_t) q * A.out_nb1 + (int64_t) h * HD;
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int k = 0; k < NT; k++) o[(g + 4 * r) * NT + k] = (float) acc[k][r];
+    }
+    item += gridDim.x;
+    } while (PT == 0 && item < n_row_tiles * A.n_head_kv);
 }
 
-static int apf_static_lds_of(int hd) {
-    return hd == 64 ? apf_static_lds<64>() : hd == 96 ? apf_static_lds<96>() : apf_static_lds<128>();
-}
-
+// positions up to which any batch of more than four queries comes here (the multi-query kernels are
+// the better ones past it for few queries: GQA, 70 queries over 2570 positions 227 us for the block, 228 here)
 int attn_prefill_max_kv(int hd) {
-    if (hd != 64 && hd != 96 && hd != 128) return 0;
-    const int rows = (max_lds_per_block() - apf_static_lds_of(hd)) / (APF_Q * (int) sizeof(float)) - 4;
-    return std::min(rows / APF_CHUNK * APF_CHUNK, APF_MAX_CHUNKS * APF_CHUNK);
+    return hd == 64 ? 2368 : hd == 96 ? 2240 : hd == 128 ? 2176 : 0;
+}
+
+static int64_t apf_items(int n_q, int n_head, int n_head_kv) {
+    return ((int64_t) n_q * (n_head / n_head_kv) + APF_ROWS - 1) / APF_ROWS * n_head_kv;
+}
+
+// Past attn_prefill_max_kv a workgroup has a CU to itself for most of a launch, so the time goes in whole
+// rounds of one workgroup per CU, while the multi-query kernels' time goes with the queries. The line lies
+// where the last round leaves a quarter of the CUs idle; the block in us, multi-query / this kernel:
+// GQA 32 heads over 8292 positions, 100 queries (200 workgroups) 534 / 504; 160 over 8352 (320) 817 / 904;
+// 200 over 8392 (400) 983 / 916; 640 over 8832 (1280) 3106 / 2265; 100 over 4000 327 / 296; 200 over 2700
+// 460 / 369; 24 heads over 5100, 100 queries (152) 314 / 353, 160 over 5160 (240) 460 / 363.
+bool attn_prefill_long_ok(int n_kv, int n_q, int n_head, int n_head_kv) {
+    const int64_t items = apf_items(n_q, n_head, n_head_kv), rounds = (items + APF_CUS - 1) / APF_CUS;
+    return n_q > ATT_DECODE_MAX_Q && n_kv <= 16 * APF_MAX_TILES && n_head / n_head_kv <= 8 &&
+           items * 4 >= rounds * APF_CUS * 3;
+}
+
+// How a launch holds its scores: pt tiles of each of `waves` waves in registers (pt = 0: in scratch).
+// Registers are the faster place (the block's time in us, scratch / registers: Phi-3 heads, 512 queries
+// over 512 positions 214 / 194; GQA, 640 over 640 281 / 260; 300 over 1800 373 / 355; 1000 over 4001
+// 1600 / 1549) while there are more workgroups than CUs. Fewer leave a CU to one workgroup, and then 8
+// waves that share its tiles beat 4 (GQA, 64 queries over 564 133 / 138; 8 over 1508 120 / 137), except
+// over rows so short that most of the 8 have nothing (Phi-3 heads, 64 over 64 76 / 72).
+struct apf_plan { int pt, waves; };
+static apf_plan apf_plan_of(int n_kv, int64_t items, bool scratch) {
+    if (n_kv > APF_REG_KV || (scratch && items <= APF_CUS && n_kv > 256)) return apf_plan{ 0, 8 };
+    if (n_kv <= 16 * 8 * 4) return apf_plan{ 8, 4 };
+    if (n_kv <= 16 * 16 * 4) return apf_plan{ 16, 4 };
+    return apf_plan{ 32, n_kv <= 16 * 32 * 4 ? 4 : 8 };
+}
+
+static int64_t apf_block_bytes(int n_kv) { return (int64_t) ((n_kv + 15) / 16) * WAVE * (int64_t) sizeof(f32x4); }
+
+// one block's scores for each of the blocks of a launch, which then takes several row tiles per block: two
+// blocks per CU, or (fixed: an arena that cannot grow) no more than what 64 queries take in the
+// multi-query kernels, and none where the registers do
+int64_t attn_prefill_scratch_bytes(int n_kv, int n_q, int n_head, int n_head_kv, bool fixed) {
+    const int64_t items = apf_items(n_q, n_head, n_head_kv);
+    if (apf_plan_of(n_kv, items, !fixed).pt) return 0;
+    return std::min<int64_t>(items, fixed ? std::min(8 * n_head, APF_MAX_BLOCKS) : APF_MAX_BLOCKS) * apf_block_bytes(n_kv);
+}
+
+template <int HD, int PT, int WAVES>
+static void launch_attn_prefill_t(const attn_launch & A, int64_t blocks, hipStream_t st) {
+    const dim3 grid((unsigned) blocks);
+    if (A.p_f32) launch((attn_prefill_kernel<HD, PT, WAVES, true>), grid, dim3(64 * WAVES), 0, st, A);
+    else launch((attn_prefill_kernel<HD, PT, WAVES, false>), grid, dim3(64 * WAVES), 0, st, A);
 }
 
 template <int HD>
 static void launch_attn_prefill_hd(const attn_launch & A, hipStream_t st) {
-    const size_t lds = std::max((size_t) APF_Q * apf_row_stride(A.n_kv) * sizeof(float), (size_t) 2 * APF_Q * HD * sizeof(double));
-    if (lds + apf_static_lds<HD>() > 65536) {
-        HIP_CHECK(hipFuncSetAttribute((const void *) attn_prefill_kernel<HD>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
-    }
-    launch(attn_prefill_kernel<HD>, dim3(A.n_head, (A.n_q + APF_Q - 1) / APF_Q), dim3(ATT_THREADS), lds, st, A);
+    const int64_t items = apf_items(A.n_q, A.n_head, A.n_head_kv);
+    if (items > INT32_MAX) HIP_ABORT("attn prefill: %d queries", A.n_q);
+    const apf_plan P = apf_plan_of(A.n_kv, items, A.scratch != nullptr);
+    if (P.pt == 0) {
+        const int64_t blocks = std::min(items, A.scratch_bytes / apf_block_bytes(A.n_kv));
+        if (!A.scratch || blocks < 1) HIP_ABORT("attn prefill: scratch too small");
+        launch_attn_prefill_t<HD, 0, 8>(A, blocks, st);
+    } else if (P.pt == 8) launch_attn_prefill_t<HD, 8, 4>(A, items, st);
+    else if (P.pt == 16) launch_attn_prefill_t<HD, 16, 4>(A, items, st);
+    else if (P.waves == 4) launch_attn_prefill_t<HD, 32, 4>(A, items, st);
+    else launch_attn_prefill_t<HD, 32, 8>(A, items, st);
 }
 
 void launch_attn_prefill(const attn_launch & A, hipStream_t st) {
-    if (A.n_q < 1 || A.n_kv < 1 || A.n_kv > attn_prefill_max_kv(A.hd)) HIP_ABORT("attn prefill: n_kv %d out of range", A.n_kv);
-    if (A.n_head % A.n_head_kv) HIP_ABORT("attn prefill: n_head %% n_head_kv");
-    if (A.out_q.qs) HIP_ABORT("attn prefill: no quantized output");
+    if (A.n_head_kv < 1 || A.n_head % A.n_head_kv) HIP_ABORT("attn prefill: n_head %% n_head_kv");
+    if (A.n_q < 1 || A.n_kv < 1 || (A.n_kv > attn_prefill_max_kv(A.hd) && !attn_prefill_long_ok(A.n_kv, A.n_q, A.n_head, A.n_head_kv))) {
+        HIP_ABORT("attn prefill: n_kv %d out of range", A.n_kv);
+    }
+    if (A.out_q.qs || A.out_q8k.set() || A.p_f32 != A.skip_masked) HIP_ABORT("attn prefill: no quantized output, flash_attn_ext's two flags together");
     if (((uintptr_t) A.k | (uintptr_t) A.v) % 16 || A.k_nb1 % 8 || A.k_nb2 % 8 || A.v_nb1 % 8 || A.v_nb2 % 8) {
         HIP_ABORT("attn prefill: K and V rows must be 16-byte aligned");
     }

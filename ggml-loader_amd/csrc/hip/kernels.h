@@ -498,9 +498,13 @@ int64_t attn_scratch_bytes(int n_kv, int n_q, int n_head, int hd);
 // RoPE folded in only for n_q <= 4)
 constexpr int ATT_DECODE_MAX_Q = 64;
 void launch_attn_decode(const attn_launch & A, hipStream_t st);
-// n_q > 4 (prefill): one workgroup per (16-query tile, head), a row's scores in LDS (no scratch, no
-// quantized output); n_kv up to attn_prefill_max_kv(hd), 0 for an unsupported head dim
+// n_q > 4 (prefill): one workgroup per (KV head, 16 of its (query, head) rows); no quantized output. n_kv up
+// to attn_prefill_max_kv(hd), 0 for an unsupported head dim
 int attn_prefill_max_kv(int hd);
+// longer rows, for batches of many queries. Scratch: attn_prefill_scratch_bytes (0: none; fixed: the
+// caller's memory cannot grow, ask for as little as works)
+bool attn_prefill_long_ok(int n_kv, int n_q, int n_head, int n_head_kv);
+int64_t attn_prefill_scratch_bytes(int n_kv, int n_q, int n_head, int n_head_kv, bool fixed);
 void launch_attn_prefill(const attn_launch & A, hipStream_t st);
 
 // ---- token sampling (k_sample.hip) ----

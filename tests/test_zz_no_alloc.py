@@ -123,6 +123,16 @@ def test_static_compute_matches_graph_compute(hip, n_new):
         assert probe[0] == probe[1], (n_kv, n_new, probe)
 
 
+def test_static_compute_of_query_batches(hip):
+    # a batch whose attention scores the growing arena keeps in scratch: in registers here
+    d = layer_inputs(700, 12)
+    st_a, ref = compute(hip, d, static=False)
+    st_b, got = compute(hip, d, static=True)
+    assert st_a == 0 and st_b == 0
+    for a, b in zip(ref, got):
+        assert np.array_equal(a, b)
+
+
 def test_static_compute_rejects_oversized_scratch(hip):
     # 64 queries x 32 heads x 8192 positions of f32 scores alone exceed the static array
     big = layer_inputs(8192, 64, hd=128, n_head=32, n_head_kv=8, seed=3)
