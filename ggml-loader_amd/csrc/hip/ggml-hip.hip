@@ -1218,9 +1218,14 @@ private:
         const int64_t cols = mm->src[1]->ne[1];
         return cols >= GEMM_MIN_COLS || (cols >= GEMM_WIDE_MIN_COLS && mm->src[0]->ne[1] >= GEMM_WIDE_MIN_ROWS);
     }
+    // narrower Q4_0 / Q8_0 products with enough 16 x 16 tiles (GEMM_MIN_TILES)
+    static bool gemm_tiles(const ggml_tensor * mm) {
+        const int64_t cols = mm->src[1]->ne[1], rows = mm->src[0]->ne[1];
+        return cols > 16 && (rows + 15) / 16 * ((cols + 15) / 16) >= GEMM_MIN_TILES;
+    }
     // a Q4_0 / Q8_0 mul_mat over a prefill-width batch: the int8-MFMA GEMM (same floats as the GEMV)
     bool gemm_route(const ggml_tensor * mm) const {
-        return mm->op == GGML_OP_MUL_MAT && gemm_wide(mm) && !is_kquant(mm->src[0]->type) && gemv_capable(mm) &&
+        return mm->op == GGML_OP_MUL_MAT && (gemm_wide(mm) || gemm_tiles(mm)) && !is_kquant(mm->src[0]->type) && gemv_capable(mm) &&
                gemm_supported(mm->src[0]->type, mm->src[0]->ne[0], mm->src[0]->ne[1]) &&
                (mm->nb[1] / sizeof(float)) % 4 == 0 && ((uintptr_t) mm->data) % 16 == 0 &&
                (is_repacked(mm->src[0]->type) || ((uintptr_t) mm->src[0]->data) % 16 == 0);
@@ -1463,8 +1468,13 @@ private:
         const int64_t n_tok = by_id ? ids->ne[1] : ncols;
         const int mc_nc = by_id ? moe_cols_per_item((int) ids->ne[0], (int) n_tok, (int) n->src[0]->ne[2],
                                                     kq ? MOE_GROUP_MAX_COLS : GEMV_MC_MAX_COLS) : 0;
-        const bool mc = !kq && fuse(FUSE_MC) && n_tok >= 2 && gemv_mc_fits(wtype, (int) K, false, mc_nc) &&
-                        (gate < 0 || gemv_mc_fits(wtype, (int) K, true, mc_nc));
+        const bool multi = !kq && fuse(FUSE_MC) && n_tok >= 2;
+        const bool mc_fits = multi && gemv_mc_fits(wtype, (int) K, false, mc_nc) && (gate < 0 || gemv_mc_fits(wtype, (int) K, true, mc_nc));
+        // Q4_0 / Q8_0 on the matrix cores, unless there are so few columns (per expert) that the vector ALU
+        // is the faster one
+        bool mmq = multi && (by_id ? mc_nc >= MM_Q_MIN_ITEM : n_tok >= MM_Q_MIN_COLS || !mc_fits);
+        for (int j : group) mmq = mmq && mm_q_supported(wtype, K, g_->nodes[j]->src[0]->ne[1]);
+        const bool mc = mmq || mc_fits;
         const auto nz = norm_.find(x);
         gemv_norm pro{};
         const act_entry * xa = nullptr;
@@ -1594,6 +1604,7 @@ private:
         const expert_groups * G = (mc || kq) && by_id ? &expert_groups_of(ids, (int) n->src[0]->ne[2], mc_nc, wtype) : nullptr;
         auto run = [&](const gemv_launch & X) {
             if (kq) launch_mm_kq(X, G, st_);
+            else if (mmq) launch_mm_q(X, G, st_);
             else if (mc) launch_gemv_mc(X, G, G ? (int) n_tok : X.ncols, st_);
             else launch_gemv(X, st_);
         };

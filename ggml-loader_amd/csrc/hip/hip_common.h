@@ -13,7 +13,8 @@
 // Activation ("x") operands of the integer dots are quantized by this backend into:
 //     q8 for Q4_0/Q8_0 weights: int8 qs[K], float d[K/32] (the fp16-rounded block scale, as
 //         ggml's Q8_0 stores it), int32 s[K/32] (sum of the block's int8 values)
-//     q8K for Q4_K weights:    int8 qs[K], float d[K/256], int16 bsums[K/16]
+//     q8K for K-quant weights: int8 qs[K], float d[K/256], int16 bsums[K/16], or for several columns
+//                              the x16 form (q8k_act::x16 in kernels.h)
 #pragma once
 
 #include <hip/hip_runtime.h>

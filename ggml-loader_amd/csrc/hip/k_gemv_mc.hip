@@ -1,6 +1,6 @@
 // k_gemv_mc.hip — quantized GEMV over several activation columns per workgroup: each weight row
-// block is read once for up to GEMV_MC_MAX_COLS columns (multi-token decode steps, prompts too
-// short for the GEMM) and, for ggml_mul_mat_id, once for all the tokens routed to
+// block is read once for up to GEMV_MC_MAX_COLS columns (Q4_0 / Q8_0 steps of two or three tokens, and
+// rows that k_mm_q.hip does not take) and, for ggml_mul_mat_id, once for all the tokens routed to
 // its expert — the batched expert grouping of the reference's MoE engine (build_prefill_lists /
 // matmul_batch, qwen_model.c:742-772, 862-939), here over the expert lists that moe_group_kernel
 // builds on the device from the routing ids.

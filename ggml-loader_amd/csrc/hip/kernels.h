@@ -142,6 +142,10 @@ constexpr int GEMM_MIN_COLS = 64;   // narrower products stay on the GEMV, excep
 // activation once per 16-row workgroup
 constexpr int GEMM_WIDE_MIN_COLS = 16;
 constexpr int64_t GEMM_WIDE_MIN_ROWS = 65536;
+// and more than one 16-column tile takes it from this many 16 x 16 tiles (us, Q4_0, k_mm_q.hip / GEMM): 3072 x
+// 8192 by 32 columns (1024 tiles) 21.0 / 22.9, by 48 (1536) 29.1 / 23.2; 3072 x 12288 by 17 (1536) 28.9 / 25.9;
+// 3072 x 32064 by 12 (one tile of columns) 32.1 / 37.1, by 17 63.9 / 37.4; 4096 x 4096 by 63 (1024) 24.5 / 28.6
+constexpr int64_t GEMM_MIN_TILES = 1536;
 
 struct gemm_launch {
     int             type;      // GGML_TYPE_Q4_0 / Q8_0
@@ -278,10 +282,18 @@ void mm_dispatch_q5_k(mm_shape s, const gemv_launch & L, const expert_groups * G
 void mm_dispatch_q6_k(mm_shape s, const gemv_launch & L, const expert_groups * G, hipStream_t st);
 // most columns of a grouped mul_mat_id's item
 constexpr int MOE_GROUP_MAX_COLS = 32;
-void launch_mm_kq(const gemv_launch & L, const expert_groups * G, hipStream_t st);
-void mm_dispatch_q4_k(mm_shape s, const gemv_launch & L, const expert_groups * G, int lds_cols, hipStream_t st);
-void mm_dispatch_q5_k(mm_shape s, const gemv_launch & L, const expert_groups * G, int lds_cols, hipStream_t st);
-void mm_dispatch_q6_k(mm_shape s, const gemv_launch & L, const expert_groups * G, int lds_cols, hipStream_t st);
+// Q4_0 / Q8_0 products of several Q8_0 columns on the matrix cores (k_mm_q.hip): dense, or a mul_mat_id's
+// columns grouped by expert in items of up to 16 (G), with the SwiGLU and residual epilogues
+bool mm_q_supported(int type, int64_t K, int64_t n_rows);
+// dense products of fewer columns go to gemv_mc (us, k_gemv_mc.hip / k_mm_q.hip: Q4_0 8192 x 3072 by 2 columns 13.0 / 17.3,
+// by 3 13.5 / 17.4, by 4 19.6 / 17.5; 3072 x 8192 11.4 / 12.3, 12.5 / 12.8, 13.5 / 12.9; Q8_0 8192 x 3072 by 2
+// 15.4 / 18.3, by 4 20.6 / 18.6)
+constexpr int MM_Q_MIN_COLS = 4;
+// and routed ones whose items hold fewer (a MoE layer in us, gemv_mc / mm_q: Q4_0 2048 x 768, 8 of 128 experts,
+// 16 tokens (items of 2 columns) 94 / 163, 56 (4) 189 / 262, 64 (8) 308 / 235, 200 (16) 1004 / 312; Q8_0 4 of 64 experts, 48 (4)
+// 114 / 164, 64 (8) 178 / 151)
+constexpr int MM_Q_MIN_ITEM = 8;
+void launch_mm_q(const gemv_launch & L, const expert_groups * G, hipStream_t st);
 // L.norm's prologue for L.ncols columns of L.K, written once to q8 (Q4_0/Q8_0 consumers) or q8k (Q4_K)
 void launch_act_quant(const gemv_launch & L, const q8_act & q8, const q8k_act & q8k, hipStream_t st);
 // consumers with more rows than this get the activation quantized once instead of per workgroup
