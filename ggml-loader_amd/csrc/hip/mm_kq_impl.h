@@ -41,6 +41,8 @@
 
 #include "ggml.h"
 
+#include <type_traits>
+
 namespace mm_kq_detail {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -439,10 +441,14 @@ __device__ __forceinline__ void store_out(const mm_kargs & A, const mm_tile & T,
 }
 
 // 16 bytes per lane from base + off straight into LDS: lane i's land at dst + 16 i (base, dst uniform)
-__device__ __forceinline__ void to_lds(const uint8_t * base, uint32_t off, uint8_t * dst) {
+template <typename OFF>
+__device__ __forceinline__ void to_lds(const uint8_t * base, OFF off, uint8_t * dst) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *) (base + off),
                                      (__attribute__((address_space(3))) void *) dst, 16, 0, 0);
 }
+
+// the shapes that a grouped launch may take (mm_shape_of)
+constexpr bool mm_groups(int wr, int wc, int nt) { return wr == 4 && wc == 1 && nt <= 2; }
 
 // WR x WC waves: WR groups of 16 rows, WC groups of 16 NT columns. Two LDS buffers of one super-block
 // of the workgroup's column groups, filled by direct global -> LDS loads (a group's super-block is
@@ -453,7 +459,9 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void mm_kq_kernel(const mm_kargs A
     const mm_kargs & A = kernargs_prefetched(A_);
     const gemv_launch & L = A.L;
     constexpr int WAVES = WR * WC, COLS = 16 * NT * WC, BM = 16 * WR, G = NT * WC;
-    constexpr int WPG = WAVES % G == 0 ? WAVES / G : 0;          // waves per column group (0: dense only)
+    constexpr int WPG = WAVES % G == 0 ? WAVES / G : 0;          // waves per column group (0: not whole)
+    constexpr bool GROUPS = mm_groups(WR, WC, NT);
+    static_assert(!GROUPS || WPG > 0, "a grouped launch's waves read the columns of one group");
     __shared__ __align__(16) uint8_t s_x0[G * X16_BYTES];
     __shared__ __align__(16) uint8_t s_x1[G * X16_BYTES];
     const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x / WAVE);
@@ -463,15 +471,16 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void mm_kq_kernel(const mm_kargs A
     const int r0 = T.rt * BM - A.row_begin[T.mi] + 16 * (wave % WR);
 
     // this wave's pieces: those of one column group, or every WAVES-th of all. Grouped, each lane
-    // reads its own column's units (columns past the end repeat the last one); dense, a group's
-    // pieces are contiguous (groups past the end repeat the last one)
+    // reads its own column's units (columns past the end repeat the last one), at 64-bit offsets: the
+    // x16 form of a large routed batch passes 4 GiB. Dense, a group's pieces are contiguous (groups
+    // past the end repeat the last one)
     const int64_t gstride = (int64_t) nsb * X16_BYTES;
     const int ng = (T.first + T.ncols + 15) / 16 - T.first / 16;
     const uint8_t * xbase = (const uint8_t *) L.xq;
-    uint32_t xoff = lane * 16;
-    if (WPG && A.g.cols) {
+    std::conditional_t<GROUPS, int64_t, uint32_t> xoff = lane * 16;
+    if (GROUPS && A.g.cols) {
         const int xc = x_column(A, T, min(16 * (wave / (WPG ? WPG : 1)) + c, T.ncols - 1));
-        xoff = (uint32_t) (xc / 16) * (uint32_t) gstride + (xc % 16) * 16 + q * 256;
+        xoff = (xc / 16) * gstride + (xc % 16) * 16 + q * 256;
     } else {
         xbase += (T.first / 16) * gstride;
     }
@@ -479,7 +488,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void mm_kq_kernel(const mm_kargs A
         const uint8_t * src = xbase + (int64_t) sb * X16_BYTES;
         if constexpr (WPG > 0) {
             const int g = wave / WPG;
-            if (!A.g.cols) src += min(g, ng - 1) * gstride;
+            if (!GROUPS || !A.g.cols) src += min(g, ng - 1) * gstride;
 #pragma unroll
             for (int i = 0; i < (X16_PIECES + WPG - 1) / WPG; i++) {
                 const int j = wave % WPG + i * WPG;
@@ -685,6 +694,7 @@ inline void mm_grid(mm_kargs & a, const gemv_launch & L, const expert_groups * G
 
 template <int TYPE, int WR, int WC, int NT>
 void mm_launch(const gemv_launch & L, const expert_groups * G, hipStream_t st) {
+    if (G && !mm_groups(WR, WC, NT)) HIP_ABORT("mm_kq: a %d x %d tile takes no expert groups", 16 * WR, 16 * NT * WC);
     mm_kargs a{};
     mm_grid(a, L, G, 16 * WR, 16 * NT * WC);
     launch(mm_kq_kernel<TYPE, WR, WC, NT>, dim3((unsigned) (a.n_rt * a.n_ct)), dim3(64 * WR * WC), 0, st, a);

@@ -77,3 +77,23 @@ def test_kquant_expert_columns(hip, cpu, qtype, n_embd, ff, E, k, n_tok):
 
     a, b = run_on(hip, build), run_on(cpu, build)
     assert np.array_equal(a, b), rel_err(a, b)
+
+
+def test_kquant_expert_columns_past_4_gib(hip, cpu):
+    """Routed columns whose quantized form passes 4 GiB (columns * K above 1.9e9): the last tokens are
+    read past that offset."""
+    K, N, E, T, R, last = 32768, 64, 2, 58300, 200, 60      # 2.25 bytes a value: 2**32 is at token 58256
+    r = rng(31)
+    rows = r.standard_normal((R, K)).astype(np.float32)
+    pick = r.integers(0, R, T).astype(np.int32)              # token t is row pick[t]
+    ids = r.integers(0, E, (T, 1)).astype(np.int32)
+    w = qweight(gl.Q4_K, K, E * N, 32)
+
+    def build(g, pick, ids):
+        x = g.get_rows(g.tensor(gl.F32, K, R, data=rows), g.tensor(gl.I32, len(pick), data=pick))
+        x = g.reshape_3d(x, K, 1, len(pick))
+        return g.mul_mat_id(g.tensor(gl.Q4_K, K, N, E, data=w), x, g.tensor(gl.I32, 1, len(ids), data=ids))
+
+    a = run_on(hip, lambda g: build(g, pick, ids)).reshape(T, N)
+    b = run_on(cpu, lambda g: build(g, pick[-last:], ids[-last:])).reshape(last, N)
+    assert np.array_equal(a[-last:], b), rel_err(a[-last:], b)
