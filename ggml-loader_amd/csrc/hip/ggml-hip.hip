@@ -169,6 +169,13 @@ planes planes_of(const ggml_tensor * t) {
     return p;
 }
 
+// the planes of a Q4_0 / Q8_0 tensor as the matrix-core kernels load them: 16-byte pieces of quants, and
+// (scales) four F16 scales at a time. A view may start at any block, and so at any scale.
+bool planes_aligned(const ggml_tensor * t, bool scales) {
+    const planes p = planes_of(t);
+    return (uintptr_t) (p.qs + p.first_block * qs_bytes_of(t->type)) % 16 == 0 && (!scales || (uintptr_t) (p.d + p.first_block) % 8 == 0);
+}
+
 q6k_planes q6k_of(const planes & p) { return q6k_planes{ p.qs, p.qh, p.sc, p.d }; }
 
 void repack_blocks(const ggml_tensor * t, const planes & p, const uint8_t * raw, int64_t nblocks, int64_t first, hipStream_t st) {
@@ -1227,8 +1234,7 @@ private:
     bool gemm_route(const ggml_tensor * mm) const {
         return mm->op == GGML_OP_MUL_MAT && (gemm_wide(mm) || gemm_tiles(mm)) && !is_kquant(mm->src[0]->type) && gemv_capable(mm) &&
                gemm_supported(mm->src[0]->type, mm->src[0]->ne[0], mm->src[0]->ne[1]) &&
-               (mm->nb[1] / sizeof(float)) % 4 == 0 && ((uintptr_t) mm->data) % 16 == 0 &&
-               (is_repacked(mm->src[0]->type) || ((uintptr_t) mm->src[0]->data) % 16 == 0);
+               (mm->nb[1] / sizeof(float)) % 4 == 0 && ((uintptr_t) mm->data) % 16 == 0 && planes_aligned(mm->src[0], false);
     }
     bool gemm_consumer(int u) const {
         for (int j : users_[u]) if (gemm_route(g_->nodes[j])) return true;
@@ -1473,7 +1479,10 @@ private:
         // Q4_0 / Q8_0 on the matrix cores, unless there are so few columns (per expert) that the vector ALU
         // is the faster one
         bool mmq = multi && (by_id ? mc_nc >= MM_Q_MIN_ITEM : n_tok >= MM_Q_MIN_COLS || !mc_fits);
-        for (int j : group) mmq = mmq && mm_q_supported(wtype, K, g_->nodes[j]->src[0]->ne[1]);
+        for (int j : group) {
+            const ggml_tensor * w = g_->nodes[j]->src[0];
+            mmq = mmq && mm_q_supported(wtype, K, w->ne[1]) && planes_aligned(w, true);
+        }
         const bool mc = mmq || mc_fits;
         const auto nz = norm_.find(x);
         gemv_norm pro{};

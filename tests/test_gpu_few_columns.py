@@ -103,3 +103,25 @@ def test_few_columns_routed(hip, cpu, qtype, n_tok):
                              g.tensor(qtype, ff, n_embd, E, data=wd), k, g.tensor(gl.F32, n_embd, n_tok, data=res))
 
     same(hip, cpu, build)
+
+
+@pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("first", [1, 2, 4])
+@pytest.mark.parametrize("K,N,ncols", [
+    (384, 100, 9),
+    (640, 4100, 16),     # a 16 x 16 tile per wave
+    (256, 12288, 20),    # the GEMM
+    (13824, 40, 5),      # too long for the vector kernel's LDS: one column at a time unless aligned
+])
+def test_few_columns_weight_view(hip, cpu, qtype, first, K, N, ncols):
+    """Rows that begin at any block of a larger tensor, so that their scales are aligned to 2 bytes."""
+    r = np.random.default_rng(N + first)
+    blocks = quantize((r.standard_normal((1, K * N + 5 * 32)) * 0.05).astype(np.float32), qtype, impl="product")
+    x = r.standard_normal((ncols, K)).astype(np.float32)
+    row = K // 32 * {gl.Q4_0: 18, gl.Q8_0: 34}[qtype]
+
+    def build(g):
+        w = g.view_2d(g.tensor(qtype, K * N + 5 * 32, data=blocks), K, N, row, first * (row // (K // 32)))
+        return g.mul_mat(w, g.tensor(gl.F32, K, ncols, data=x))
+
+    same(hip, cpu, build)
