@@ -609,9 +609,12 @@ private:
         return e;
     }
     // a product of several columns with K-quant weights: the matrix-core kernel (launch_mm_kq), which
-    // reads the x16 form
+    // reads the x16 form, unless the expert lists would not hold its experts
     static bool kq_multi(const ggml_tensor * mm) {
-        return is_kquant(mm->src[0]->type) && (mm->op == GGML_OP_MUL_MAT_ID ? mm->src[2]->ne[1] : mm->src[1]->ne[1]) >= 2;
+        const ggml_tensor * w = mm->src[0];
+        if (!is_kquant(w->type)) return false;
+        if (mm->op == GGML_OP_MUL_MAT_ID) return mm->src[2]->ne[1] >= 2 && w->ne[2] <= MOE_GROUP_MAX_EXPERTS;
+        return mm->src[1]->ne[1] >= 2;
     }
     // the quantized form of its activation that a mul_mat / mul_mat_id reads (act_entry::kind; 0: none)
     static int act_kind_of(const ggml_tensor * mm) { return kq_multi(mm) ? 3 : dot_kind(mm->src[0]->type); }
@@ -1312,10 +1315,13 @@ private:
             q8k_act q8k{};
             if (fuse(FUSE_ACTQ) && m->ne[0] % 256 == 0 && is_2d_contig(m)) {
                 bool kq = false, other = false;
+                int kind = 0;                    // the form that the readers take, the same for all
                 std::vector<const ggml_tensor *> readers = { m };
                 auto kq_reader = [&](const ggml_tensor * un, const ggml_tensor * src) {
-                    return (un->op == GGML_OP_MUL_MAT || un->op == GGML_OP_MUL_MAT_ID) && un->src[1] == src &&
-                           un->src[0] != src && dot_kind(un->src[0]->type) == 2;
+                    if ((un->op != GGML_OP_MUL_MAT && un->op != GGML_OP_MUL_MAT_ID) || un->src[1] != src || un->src[0] == src ||
+                        dot_kind(un->src[0]->type) != 2 || (kind && act_kind_of(un) != kind)) return false;
+                    kind = act_kind_of(un);
+                    return true;
                 };
                 for (int j : users_[rn->second.mul]) {
                     const ggml_tensor * un = g_->nodes[j];
@@ -1334,7 +1340,7 @@ private:
                     }
                 }
                 if (kq && !other) {
-                    act_entry e = alloc_act(m->ne[1] >= 2 ? 3 : 2, m->ne[0], m->ne[1]);
+                    act_entry e = alloc_act(kind, m->ne[0], m->ne[1]);
                     q8k = e.q8k;
                     for (const ggml_tensor * r : readers) act_[r] = e;
                 }
@@ -1442,7 +1448,7 @@ private:
                 const ggml_tensor * m = g_->nodes[j];
                 if (done_[j] || m->op != n->op || m->src[1] != x || (by_id && m->src[2] != ids)) continue;
                 if (attn_.count(j)) continue;
-                if (m->src[0]->type != wtype || m->src[0]->ne[0] != K || !gemv_capable(m)) continue;
+                if (m->src[0]->type != wtype || m->src[0]->ne[0] != K || act_kind_of(m) != act_kind_of(n) || !gemv_capable(m)) continue;
                 if ((int) group.size() == GEMV_MAX_MATS) break;
                 group.push_back(j);
             }

@@ -147,7 +147,7 @@ void launch_gemv_mc(const gemv_launch & L, const expert_groups * G, int max_cols
 
 void launch_moe_group(const int32_t * ids, int64_t ids_stride, int n_slots, int n_tok, int n_experts, const expert_groups & g,
                       hipStream_t st) {
-    if (n_experts < 1 || n_experts > 4096 || n_slots < 1 || n_tok < 1) HIP_ABORT("moe_group: %d experts", n_experts);
+    if (n_experts < 1 || n_experts > MOE_GROUP_MAX_EXPERTS || n_slots < 1 || n_tok < 1) HIP_ABORT("moe_group: %d experts", n_experts);
     const int ncol = n_slots * n_tok;
     if (g.nc < 1 || g.nc > MOE_GROUP_MAX_COLS || g.max_items < std::min(n_experts, ncol) + (ncol + g.nc - 1) / g.nc) {
         HIP_ABORT("moe_group: %d items of %d columns cannot hold %d columns", g.max_items, g.nc, ncol);

@@ -280,8 +280,8 @@ void launch_mm_kq(const gemv_launch & L, const expert_groups * G, hipStream_t st
 void mm_dispatch_q4_k(mm_shape s, const gemv_launch & L, const expert_groups * G, hipStream_t st);
 void mm_dispatch_q5_k(mm_shape s, const gemv_launch & L, const expert_groups * G, hipStream_t st);
 void mm_dispatch_q6_k(mm_shape s, const gemv_launch & L, const expert_groups * G, hipStream_t st);
-// most columns of a grouped mul_mat_id's item
-constexpr int MOE_GROUP_MAX_COLS = 32;
+// most columns of a grouped mul_mat_id's item, and most experts (two counters each in a workgroup's LDS)
+constexpr int MOE_GROUP_MAX_COLS = 32, MOE_GROUP_MAX_EXPERTS = 4096;
 // Q4_0 / Q8_0 products of several Q8_0 columns on the matrix cores (k_mm_q.hip): dense, or a mul_mat_id's
 // columns grouped by expert in items of up to 16 (G), with the SwiGLU and residual epilogues
 bool mm_q_supported(int type, int64_t K, int64_t n_rows);

@@ -97,3 +97,21 @@ def test_kquant_expert_columns_past_4_gib(hip, cpu):
     a = run_on(hip, lambda g: build(g, pick, ids)).reshape(T, N)
     b = run_on(cpu, lambda g: build(g, pick[-last:], ids[-last:])).reshape(last, N)
     assert np.array_equal(a[-last:], b), rel_err(a[-last:], b)
+
+
+@pytest.mark.parametrize("qtype", [gl.Q5_K, gl.Q6_K])
+def test_kquant_many_experts(hip, cpu, qtype):
+    """More experts than the expert lists hold: each column reads its own."""
+    K, N, E, k, T = 256, 8, 4100, 2, 3
+    r = rng(41)
+    x, x2 = (r.standard_normal((T, n, K)).astype(np.float32) for n in (1, k))
+    ids = r.integers(0, E, (T, k)).astype(np.int32)
+    ids[0] = (0, E - 1)
+    w = qweight(qtype, K, E * N, 42)
+
+    def build(g):
+        wt, it = g.tensor(qtype, K, N, E, data=w), g.tensor(gl.I32, k, T, data=ids)
+        return [g.mul_mat_id(wt, g.tensor(gl.F32, K, v.shape[1], T, data=v), it) for v in (x, x2)]
+
+    for a, b in zip(run_on(hip, build), run_on(cpu, build)):
+        assert np.array_equal(a, b), rel_err(a, b)
