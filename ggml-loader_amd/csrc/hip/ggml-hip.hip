@@ -609,10 +609,13 @@ private:
         return e;
     }
     // a product of several columns with K-quant weights: the matrix-core kernel (launch_mm_kq), which
-    // reads the x16 form, unless the expert lists would not hold its experts
+    // reads the x16 form, unless the expert lists would not hold its experts or a caller placed the
+    // weights (Q6_K: their first plane) at an address that its 16-byte loads do not take
     static bool kq_multi(const ggml_tensor * mm) {
         const ggml_tensor * w = mm->src[0];
         if (!is_kquant(w->type)) return false;
+        const void * at = is_repacked(w->type) && w->view_src ? w->view_src->data : w->data;
+        if ((uintptr_t) at % 16) return false;
         if (mm->op == GGML_OP_MUL_MAT_ID) return mm->src[2]->ne[1] >= 2 && w->ne[2] <= MOE_GROUP_MAX_EXPERTS;
         return mm->src[1]->ne[1] >= 2;
     }

@@ -1,10 +1,12 @@
 """Products of several activation columns at the edges of their workgroup shapes (rows and columns
 that end inside a tile, one super-block, several chunks), dense and routed, against the oracle: the
 same floats (every kernel adds the oracle's terms in the oracle's order)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from gl import cpu_backend, gl, moe_ffn_graph, quantize, rel_err, run_on
+from gl import Graph, cpu_backend, gl, moe_ffn_graph, quantize, rel_err, run_on
 
 pytestmark = pytest.mark.gpu
 
@@ -115,3 +117,32 @@ def test_kquant_many_experts(hip, cpu, qtype):
 
     for a, b in zip(run_on(hip, build), run_on(cpu, build)):
         assert np.array_equal(a, b), rel_err(a, b)
+
+
+@pytest.mark.parametrize("qtype", [gl.Q4_K, gl.Q5_K])
+@pytest.mark.parametrize("ncols", [5, 70])
+def test_kquant_weights_at_8_bytes(hip, cpu, qtype, ncols):
+    """Weights that a caller placed 8 bytes past the buffer's alignment."""
+    core = gl.libs()["core"]
+    K, N = 512, 100
+    w = qweight(qtype, K, N, 51)
+    x = rng(52).standard_normal((ncols, K)).astype(np.float32)
+
+    def run(backend):
+        buft = C.c_void_p(core.ggml_backend_get_default_buffer_type(backend))
+        buf = C.c_void_p(core.ggml_backend_buft_alloc_buffer(buft, w.nbytes + 1024))
+        with Graph() as g:
+            wt = g.tensor(qtype, K, N, data=w)
+            core.ggml_backend_tensor_alloc(buf, wt, C.c_void_p(core.ggml_backend_buffer_get_base(buf) + 8))
+            out = g.compute(backend, g.mul_mat(wt, g.tensor(gl.F32, K, ncols, data=x)))
+        core.ggml_backend_buffer_free(buf)
+        return out
+
+    for name in ("ggml_backend_get_default_buffer_type", "ggml_backend_buft_alloc_buffer", "ggml_backend_buffer_get_base"):
+        getattr(core, name).restype = C.c_void_p
+    core.ggml_backend_get_default_buffer_type.argtypes = [C.c_void_p]
+    core.ggml_backend_buft_alloc_buffer.argtypes = [C.c_void_p, C.c_size_t]
+    core.ggml_backend_buffer_get_base.argtypes = [C.c_void_p]
+    core.ggml_backend_tensor_alloc.argtypes = [C.c_void_p, gl.T, C.c_void_p]
+    a, b = run(hip), run(cpu)
+    assert np.array_equal(a, b), rel_err(a, b)
