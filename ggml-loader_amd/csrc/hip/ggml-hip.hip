@@ -1426,6 +1426,34 @@ private:
         return std::string("gemm_") + ggml_type_name((enum ggml_type) L.type) + "_" + mm_shape_name(mm_shape_of(L, G));
     }
 
+    // node i and the other pending quantized products of its input that its launch takes along
+    std::vector<int> gemv_group(int i) const {
+        const ggml_tensor * n = g_->nodes[i], * x = n->src[1];
+        const bool by_id = n->op == GGML_OP_MUL_MAT_ID;
+        std::vector<int> group = { i };
+        if (!fuse(FUSE_GROUP)) return group;
+        const int xi = node_index(x);
+        std::vector<int> others;
+        if (xi < 0) {
+            for (int j = i + 1; j < g_->n_nodes; j++) {
+                const ggml_tensor * m = g_->nodes[j];
+                if (m->op == n->op && m->src[1] == x) others.push_back(j);
+            }
+        } else {
+            for (int j : users_[xi]) if (j != i) others.push_back(j);
+        }
+        for (int j : others) {
+            const ggml_tensor * m = g_->nodes[j];
+            if (done_[j] || m->op != n->op || m->src[1] != x || (by_id && m->src[2] != n->src[2])) continue;
+            if (attn_.count(j)) continue;
+            if (m->src[0]->type != n->src[0]->type || m->src[0]->ne[0] != n->src[0]->ne[0] || act_kind_of(m) != act_kind_of(n) ||
+                !gemv_capable(m)) continue;
+            if ((int) group.size() == GEMV_MAX_MATS) break;
+            group.push_back(j);
+        }
+        return group;
+    }
+
     // quantized GEMV for node i, grouped with the other pending mul_mats that read the same input
     void op_gemv(int i) {
         ggml_tensor * n = g_->nodes[i];
@@ -1435,27 +1463,7 @@ private:
         const ggml_tensor * ids = by_id ? n->src[2] : nullptr;
         const int64_t K = n->src[0]->ne[0];
         const int64_t ncols = by_id ? ids->ne[0] * ids->ne[1] : x->ne[1];   // launch columns
-        std::vector<int> group = { i };
-        if (fuse(FUSE_GROUP)) {
-            const int xi = node_index(x);
-            std::vector<int> others;
-            if (xi < 0) {
-                for (int j = i + 1; j < g_->n_nodes; j++) {
-                    const ggml_tensor * m = g_->nodes[j];
-                    if (m->op == n->op && m->src[1] == x) others.push_back(j);
-                }
-            } else {
-                for (int j : users_[xi]) if (j != i) others.push_back(j);
-            }
-            for (int j : others) {
-                const ggml_tensor * m = g_->nodes[j];
-                if (done_[j] || m->op != n->op || m->src[1] != x || (by_id && m->src[2] != ids)) continue;
-                if (attn_.count(j)) continue;
-                if (m->src[0]->type != wtype || m->src[0]->ne[0] != K || act_kind_of(m) != act_kind_of(n) || !gemv_capable(m)) continue;
-                if ((int) group.size() == GEMV_MAX_MATS) break;
-                group.push_back(j);
-            }
-        }
+        std::vector<int> group = gemv_group(i);
 
         // SwiGLU pair inside the group: gate -> silu -> mul(silu, up)
         const bool kq = kq_multi(n);
@@ -1707,6 +1715,11 @@ private:
         v.ne[2] = v.ne[3] = 1;
         return v;
     }
+    // node k: a dense K-quant product of several columns whose launch takes no other product along
+    bool kq_alone(int k) const {
+        const ggml_tensor * t = g_->nodes[k];
+        return t->op == GGML_OP_MUL_MAT && !attn_.count(k) && kq_multi(t) && gemv_capable(t) && gemv_group(k).size() == 1;
+    }
     bool op_swiglu(int i) {
         ggml_tensor * sn = g_->nodes[i];
         if (sn->op_params[0] != GGML_UNARY_OP_SILU) return false;
@@ -1726,12 +1739,13 @@ private:
         if (!disjoint_or_same(mn, gt) || !disjoint_or_same(mn, up)) return false;
         if (!ready(up)) {
             // separate projections: up comes after the silu. Hold the silu back (nothing launched)
-            // when the nodes before the mul are only the up projection on the prefill GEMM (no
-            // fused writes elsewhere) and views, and the projection does not write over the gate.
+            // when the nodes before the mul are only the up projection, on the prefill GEMM or in a
+            // K-quant launch of its own (of a type that is not the gate's: no fused writes elsewhere),
+            // and views, and the projection does not write over the gate.
             for (int k = i + 1; k < mj; k++) {
                 const ggml_tensor * t = g_->nodes[k];
                 if (done_[k] || is_view_op(t->op)) continue;
-                if (t != up || !gemm_route(t) || sole_user(k) != mj || !disjoint_or_same(t, gt) || t->data == gt->data) return false;
+                if (t != up || !(gemm_route(t) || kq_alone(k)) || sole_user(k) != mj || !disjoint_or_same(t, gt) || t->data == gt->data) return false;
             }
             silu_of_[mj] = i;
             return true;

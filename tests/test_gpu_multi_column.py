@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from gl import Graph, cpu_backend, gl, moe_ffn_graph, quantize, rel_err, run_on
+from test_gpu_ops import profiled
 
 pytestmark = pytest.mark.gpu
 
@@ -146,3 +147,26 @@ def test_kquant_weights_at_8_bytes(hip, cpu, qtype, ncols):
     core.ggml_backend_tensor_alloc.argtypes = [C.c_void_p, gl.T, C.c_void_p]
     a, b = run(hip), run(cpu)
     assert np.array_equal(a, b), rel_err(a, b)
+
+
+@pytest.mark.parametrize("third", [False, True])
+@pytest.mark.parametrize("gtype,utype", [(gl.Q4_K, gl.Q6_K), (gl.Q6_K, gl.Q5_K), (gl.Q4_0, gl.Q4_K)])
+def test_swiglu_of_two_types(hip, cpu, gtype, utype, third):
+    """Gate and up of different types over a prompt: silu, product and quantization in one launch, unless
+    up's launch would write a third product before the silu's turn."""
+    K, F, T = 256, 512, 70
+    x = rng(61).standard_normal((T, K)).astype(np.float32)
+    wg, wu, wd, w3 = qweight(gtype, K, F, 62), qweight(utype, K, F, 63), qweight(gl.Q4_K, F, K, 64), qweight(utype, K, 32, 65)
+
+    def build(g):
+        xt = g.tensor(gl.F32, K, T, data=x)
+        silu = g.silu(g.mul_mat(g.tensor(gtype, K, F, data=wg), xt))
+        act = g.mul(silu, g.mul_mat(g.tensor(utype, K, F, data=wu), xt))
+        outs = [g.mul_mat(g.tensor(gl.Q4_K, F, K, data=wd), act)]
+        return outs + [g.mul_mat(g.tensor(utype, K, 32, data=w3), xt)] if third else outs
+
+    a, names = profiled(hip, lambda: run_on(hip, build))
+    b = run_on(cpu, build)
+    assert ("swiglu" in names) != third, names
+    for u, v in zip(a if third else [a], b if third else [b]):
+        assert np.array_equal(u, v), rel_err(u, v)
