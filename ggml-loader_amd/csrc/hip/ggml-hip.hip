@@ -1359,7 +1359,7 @@ private:
     }
 
     // Columns per grouped workgroup: about the columns an active expert gets with uniform routing
-    // (1 - (1 - k/E)^T of the experts are active), as a power of two in [2, 16]
+    // (1 - (1 - k/E)^T of the experts are active), as a power of two from 2 to most
     static int moe_cols_per_item(int n_slots, int n_tok, int n_experts, int most) {
         const double active = n_experts * (1.0 - std::pow(1.0 - std::min(1.0, (double) n_slots / n_experts), (double) n_tok));
         const double avg = (double) n_slots * n_tok / std::max(1.0, active);
@@ -1386,7 +1386,7 @@ private:
     // The columns of a mul_mat_id grouped by expert, in items of up to nc columns (once per ids tensor,
     // nc and graph compute)
     std::map<std::pair<const ggml_tensor *, int>, expert_groups> groups_;
-    const expert_groups & expert_groups_of(const ggml_tensor * ids, int n_experts, int nc, int wtype) {
+    const expert_groups & expert_groups_of(const ggml_tensor * ids, int n_experts, int nc) {
         auto it = groups_.find({ ids, nc });
         if (it != groups_.end()) return it->second;
         const int n_slots = (int) ids->ne[0], n_tok = (int) ids->ne[1], ncol = n_slots * n_tok;
@@ -1399,7 +1399,7 @@ private:
         g.items = (int32_t *) c_.scratch.alloc((size_t) g.max_items * 3 * sizeof(int32_t));
         g.n_items = (int32_t *) c_.scratch.alloc(sizeof(int32_t));
         {
-            prof_scope ps(this, wtype == GGML_TYPE_Q5_K || wtype == GGML_TYPE_Q6_K ? "moe_group_k56" : "moe_group", 0);
+            prof_scope ps(this, "moe_group", 0);
             launch_moe_group((const int32_t *) ids->data, (int64_t) (ids->nb[1] / sizeof(int32_t)), n_slots, n_tok, n_experts, g, st_);
         }
         return groups_[{ ids, nc }] = g;
@@ -1419,7 +1419,7 @@ private:
         return rows <= GEMV_PROLOGUE_MAX_ROWS;
     }
 
-    // profile name of a prefill-width K-quant product (with its workgroup tile, e.g. gemm_q4_K_2x2);
+    // profile name of a prefill-width K-quant product (with its workgroup tile, e.g. gemm_q4_K_64x64);
     // empty for the others, which keep the GEMV names
     std::string kq_name(const gemv_launch & L, bool wide, const expert_groups * G) const {
         if (!wide || !is_kquant(L.type)) return {};
@@ -1627,7 +1627,7 @@ private:
         if (by_id && c_.timing && !route_in) n_unique_experts = distinct_ids(ids, n->src[0]->ne[2]);
         const double x_bytes = (double) (K * ggml_nrows(x) * 4) + (xa ? 0.0 : (double) (K * 4));
         // one column per workgroup, or several (mul_mat_id: the tokens routed to each expert)
-        const expert_groups * G = (mc || kq) && by_id ? &expert_groups_of(ids, (int) n->src[0]->ne[2], mc_nc, wtype) : nullptr;
+        const expert_groups * G = (mc || kq) && by_id ? &expert_groups_of(ids, (int) n->src[0]->ne[2], mc_nc) : nullptr;
         auto run = [&](const gemv_launch & X) {
             if (kq) launch_mm_kq(X, G, st_);
             else if (mmq) launch_mm_q(X, G, st_);

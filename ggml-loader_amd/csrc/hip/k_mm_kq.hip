@@ -37,10 +37,10 @@ mm_shape mm_shape_of(const gemv_launch & L, const expert_groups * G) {
 
 const char * mm_shape_name(mm_shape s) {
     switch (s) {
-        case MM_64x64: return "2x2";
-        case MM_32x64: return "1x2";
+        case MM_64x64: return "64x64";
+        case MM_32x64: return "32x64";
         case MM_64x48: return "64x48";
-        case MM_64x32: return "2x1";
+        case MM_64x32: return "64x32";
         case MM_64x16: return "64x16";
         case MM_16x16: return "16x16";
         case MM_SPLIT: return "split";

@@ -245,17 +245,18 @@ def test_gemm_subnormal_scales(hip, cpu, qtype):
     (gl.Q8_0, 128, 16400, 520, "2x4x2"),
     (gl.Q8_0, 128, 32768, 512, "4x4x2"),     # 1024 tiles of 128 x 128
     (gl.Q8_0, 256, 4096, 512, "1x2x4"),      # below both thresholds
-    (gl.Q4_K, 256, 4096, 512, "2x2"),        # 64 x 64 tiles: 512 (>= 256)
-    (gl.Q4_K, 512, 4120, 515, "2x2"),        # partial tiles, two super-blocks per row
-    (gl.Q4_K, 256, 1024, 512, "1x2"),        # 128 tiles of 64 x 64: 32 x 64 instead
-    (gl.Q5_K, 256, 4096, 512, "2x2"),
-    (gl.Q5_K, 512, 1000, 70, "1x2"),
-    (gl.Q6_K, 512, 4120, 515, "2x2"),
-    (gl.Q6_K, 256, 1024, 512, "1x2"),
+    (gl.Q4_K, 256, 4096, 512, "64x64"),      # 64 x 64 tiles: 512 (>= 256)
+    (gl.Q4_K, 512, 4120, 515, "64x64"),      # partial tiles, two super-blocks per row
+    (gl.Q4_K, 256, 1024, 512, "32x64"),      # 128 tiles of 64 x 64: 32 x 64 instead
+    (gl.Q5_K, 256, 4096, 512, "64x64"),
+    (gl.Q5_K, 512, 1000, 70, "32x64"),
+    (gl.Q6_K, 512, 4120, 515, "64x64"),
+    (gl.Q6_K, 256, 1024, 512, "32x64"),
 ])
 def test_gemm_tile_variants(hip, cpu, qtype, K, N, ncols, tile):
-    """Each workgroup tile of the prefill GEMM (the launch picks it from the tile count), pinned by
-    the profile name and bit-exact against the oracle; small K keeps the oracle cheap."""
+    """Each workgroup tile of the prefill GEMM (Q4_0, Q8_0) and of the K-quants' multi-column kernel at
+    that width (the launch picks it from the tile count), pinned by the profile name and bit-exact
+    against the oracle; small K keeps the oracle cheap."""
     w = qweight(qtype, K, N, K + 7 * N + ncols)
     x = rng(K + ncols + 5).standard_normal((ncols, K)).astype(np.float32)
 
@@ -1068,11 +1069,7 @@ def test_moe_ffn(hip, cpu, qtype, n_tok):
     # one token on the single-column Q4_K kernel: the routing runs inside the gate/up launch
     in_gemv = qtype == gl.Q4_K and n_tok == 1
     assert ("moe_route" in names) != in_gemv and ("gemv_q4_K_swiglu_route" in names) == in_gemv, names
-    if qtype in (gl.Q5_K, gl.Q6_K):
-        # no multi-column kernel for these types: each (token, slot) column reads its expert
-        assert "moe_group" not in names, names
-    else:
-        assert (n_tok >= 2) == ("moe_group" in names), names   # several tokens: experts read once for all of theirs
+    assert (n_tok >= 2) == ("moe_group" in names), names   # several tokens: experts read once for all of theirs
 
 
 @pytest.mark.parametrize("n_tok", [1, 5])
