@@ -170,3 +170,32 @@ def test_swiglu_of_two_types(hip, cpu, gtype, utype, third):
     assert ("swiglu" in names) != third, names
     for u, v in zip(a if third else [a], b if third else [b]):
         assert np.array_equal(u, v), rel_err(u, v)
+
+
+@pytest.mark.parametrize("n_tok", [5, 70])
+def test_kquant_activations_share_buffers(hip, cpu, n_tok):
+    """Activations of one size, whose quantized forms take each other's buffers once their readers are
+    launched. A SwiGLU's and a norm's, which exist in no other form, are read again by another type after
+    others came and went; one is read again through a reshape, one is an output."""
+    K, T = 512, n_tok
+    x = rng(81).standard_normal((T, K)).astype(np.float32)
+    s = (1 + 0.1 * rng(82).standard_normal(K)).astype(np.float32)
+    types = {"gate": gl.Q4_K, "up": gl.Q4_K, "a4": gl.Q4_K, "a6": gl.Q6_K, "p": gl.Q5_K, "n4": gl.Q4_K, "n5": gl.Q5_K,
+             "b4": gl.Q4_K, "b6": gl.Q6_K, "c": gl.Q6_K}
+    w = {k: qweight(t, K, K, 83 + i, std=0.05) for i, (k, t) in enumerate(types.items())}
+
+    def build(g):
+        st, xt = g.tensor(gl.F32, K, data=s), g.tensor(gl.F32, K, T, data=x)
+        wt = {k: g.tensor(t, K, K, data=w[k]) for k, t in types.items()}
+        a = g.mul(g.silu(g.mul_mat(wt["gate"], xt)), g.mul_mat(wt["up"], xt))
+        p = g.mul_mat(wt["a4"], a)
+        q = g.mul_mat(wt["p"], p)                              # p is done with
+        n = g.mul(g.rms_norm(q, 1e-5), st)
+        b = g.mul(g.mul_mat(wt["n4"], n), st)
+        r = g.mul_mat(wt["b4"], b)
+        c = g.mul(r, st)
+        out = [c, g.mul_mat(wt["c"], c), g.mul_mat(wt["a6"], a), g.mul_mat(wt["n5"], n)]
+        return out + [g.mul_mat(wt["b6"], g.reshape_2d(b, K, T)), g.mul_mat(wt["c"], g.mul(out[1], st)), g.mul_mat(wt["p"], c)]
+
+    for u, v in zip(run_on(hip, build), run_on(cpu, build)):
+        assert np.array_equal(u, v), rel_err(u, v)

@@ -806,6 +806,7 @@ def test_attention_output_accumulated_into_o_projection(hip, cpu, qtype, hd, n_h
     (gl.Q4_K, 128, 32, 4, 2400, 16),   # the MoE 16-token step: the multi-query matrix-core kernels
     (gl.Q4_K, 128, 16, 8, 300, 3),     # the four-query decode kernels
     (gl.Q6_K, 64, 8, 8, 90, 3),        # head dim 64: four heads per super-block
+    (gl.Q4_K, 128, 24, 8, 2300, 70),   # a second group of queries, after 64
 ])
 def test_attention_combination_writes_q8k(hip, cpu, qtype, hd, n_head, n_head_kv, n_kv, n_new):
     """Several queries' attention read by a K-quant O projection: the combination launch writes the
@@ -914,7 +915,7 @@ def test_attention_prefill(hip, cpu, hd, n_head, n_head_kv, n_kv, n_new, flash):
 ])
 @pytest.mark.parametrize("flash", [False, True])
 def test_attention_long_context_query_groups(hip, cpu, hd, n_head, n_head_kv, n_kv, n_new, flash):
-    """A multi-token step over more positions than the prefill kernel holds in LDS: the multi-query
+    """A multi-token step over more positions than the prefill kernel takes for so few queries: the multi-query
     decode kernels (scores and P V on the f64 matrix cores over tiles of 16 (query, head) rows,
     launches of up to 64 queries), the chain's float roundings exactly."""
     r = rng(n_kv + 7 * n_new)

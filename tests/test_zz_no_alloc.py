@@ -134,7 +134,7 @@ def test_static_compute_of_query_batches(hip):
 
 
 def test_static_compute_rejects_oversized_scratch(hip):
-    # 64 queries x 32 heads x 8192 positions of f32 scores alone exceed the static array
+    # 64 queries x 32 heads x 8192 positions: 64 MiB of f32 scores and 128 MiB of partial outputs in double
     big = layer_inputs(8192, 64, hd=128, n_head=32, n_head_kv=8, seed=3)
     st, _ = compute(hip, big, static=True)
     assert st == GGML_STATUS_ALLOC_FAILED
