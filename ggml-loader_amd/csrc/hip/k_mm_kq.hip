@@ -18,11 +18,17 @@ mm_shape mm_shape_of(const gemv_launch & L, const expert_groups * G) {
     auto tiles = [&](int cols) { return rows * ((L.ncols + cols - 1) / cols); };
     // 64 columns and more. The 64 x 64 tile decodes the weights least often; below one per CU the 32 x
     // 64 one (each wave a quarter of the columns) doubles the waves, and between one and two per CU,
-    // where some CUs would run two tiles and others one, 64 x 48 ones even that out (K = 9728, 2560
-    // rows, 512 columns: 320 tiles of 64 x 64 114.9 us, 440 of 64 x 48 86.1).
+    // where some CUs would run two tiles and others one, 64 x 48 ones even that out while they too are at
+    // most two per CU. Measured, 64x64 / 64x48, us with the quantization launch (rows x K by columns):
+    // Q4_K 288 tiles of 64 x 64 (4608 x 2560 by 256) 31.2 / 28.0, 320 (2560 x 9728 by 512) 97.8 / 85.3, 352
+    // (2816 x 2560 by 512) 33.7 / 30.5; past two 64 x 48 per CU, 384 (6144 x 2560 by 256) 31.8 / 42.4, 448
+    // (3584 x 2560 by 512) 34.2 / 44.5; Q5_K 320 112 / 99, 384 54 / 74; Q6_K 320 179 / 141, 384 54 / 63. At one per
+    // CU exactly there is nothing to even out: 4096 x 2560 by 256 Q4_K 25.2 / 27.9, Q5_K 28.4 / 31.2; Q6_K, whose 64 x
+    // 64 tile spills registers, 46.1 / 42.7.
     if (L.ncols >= 64) {
         if (tiles(64) < 256) return MM_32x64;
-        return tiles(64) < 512 && tiles(48) <= 512 ? MM_64x48 : MM_64x64;
+        const bool uneven = tiles(64) > 256 || L.type == GGML_TYPE_Q6_K;
+        return uneven && tiles(64) < 512 && tiles(48) <= 512 ? MM_64x48 : MM_64x64;
     }
     // Below 64 columns, 16 per tile. With a 64-row workgroup for every CU its four waves share the
     // staged columns. With fewer, one-wave workgroups spread over all CUs; where those are too few to

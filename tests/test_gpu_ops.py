@@ -252,6 +252,9 @@ def test_gemm_subnormal_scales(hip, cpu, qtype):
     (gl.Q5_K, 512, 1000, 70, "32x64"),
     (gl.Q6_K, 512, 4120, 515, "64x64"),
     (gl.Q6_K, 256, 1024, 512, "32x64"),
+    (gl.Q4_K, 256, 4096, 256, "64x64"),      # 256: one per CU
+    (gl.Q6_K, 256, 4096, 256, "64x48"),
+    (gl.Q5_K, 256, 4100, 256, "64x48"),      # 260
 ])
 def test_gemm_tile_variants(hip, cpu, qtype, K, N, ncols, tile):
     """Each workgroup tile of the prefill GEMM (Q4_0, Q8_0) and of the K-quants' multi-column kernel at
