@@ -31,14 +31,17 @@ mm_shape mm_shape_of(const gemv_launch & L, const expert_groups * G) {
         return uneven && tiles(64) < 512 && tiles(48) <= 512 ? MM_64x48 : MM_64x64;
     }
     // Below 64 columns, 16 per tile. With a 64-row workgroup for every CU its four waves share the
-    // staged columns. With fewer, one-wave workgroups spread over all CUs; where those are too few to
-    // keep the weights streaming, K is split over eight waves: while all its workgroups (two per CU)
-    // run at once, or for long rows. Measured (us with the quantization launch, 64x16 / 16x16 / split):
-    // Q4_K K = 2560, 9728 rows, 16 columns 14.2 / 14.2 / 16.5; Q6_K 22.2 / 19.4 / 26.4; Q4_K K = 9728,
-    // 2560 rows, 16 columns - / 32.2 / 17.7, 37 columns 33.8 / 33.2 / 24.0; Q6_K 63 columns 64.1 / 52 / 50.4;
-    // Q4_K K = 4096, 2048 rows, 16 columns - / 19 / 11.4.
+    // staged columns. With fewer, one-wave workgroups spread over all CUs; and K is split over eight waves
+    // while all those workgroups (two per CU) run at once: 128 tiles of 64 rows. Past that the split costs its LDS
+    // exchange for nothing, except over Q6_K's long rows. Measured, 64x16 / 16x16 / split, us with the
+    // quantization launch (rows x K by columns):
+    // up to 128 tiles: Q4_K 2048 x 2560 by 16 (32) 12.4 / 12.3 / 8.9, 4096 x 4096 by 16 (64) 17.1 / 16.3 / 10.4, 2560 x 9728
+    // by 37 (120) 31.6 / 32.3 / 23.0, 8192 x 2560 by 16 (128) 12.5 / 12.6 / 12.0; Q5_K 128 14.8 / 14.0 / 13.9; Q6_K 128 20.1 / 18.3 / 18.3;
+    // past it: 2560 rows by 60 (160), K = 4096 Q4_K 17.7 / 17.1 / 18.9, Q5_K 21.5 / 19.4 / 22.4, Q6_K 27.4 / 25.2 / 27.7;
+    // K = 6144 23.5 / 22.7 / 23.9, 29.1 / 26.0 / 29.8, 41.0 / 34.2 / 34.9; K = 8192 29.4 / 28.3 / 29.5, 36.7 / 32.5 / 35.6,
+    // 50.6 / 44.2 / 43.3; K = 14336 47.5 / 45.1 / 45.7, 59.8 / 52.3 / 56.9, 88.4 / 71.5 / 65.9.
     if (tiles(16) >= 256) return MM_64x16;
-    return tiles(16) <= 128 || L.K >= 4096 ? MM_SPLIT : MM_16x16;
+    return tiles(16) <= 128 || (L.type == GGML_TYPE_Q6_K && L.K >= 8192) ? MM_SPLIT : MM_16x16;
 }
 
 const char * mm_shape_name(mm_shape s) {

@@ -42,6 +42,9 @@ KQUANTS = [gl.Q4_K, gl.Q5_K, gl.Q6_K]
     (256, 16420, 17),    # a 64-row workgroup per CU, the second column tile with one column
     (256, 9000, 2),      # one-wave workgroups
     (4352, 100, 33),     # K over eight waves: three chunks, the last with one super-block
+    (256, 8190, 16),     # 128 tiles of 64 x 16: K over the waves
+    (256, 2700, 40),     # 129
+    (8192, 2690, 33),    # 129 and long rows: K over the waves for Q6_K
     (512, 4112, 250),    # 64 x 48 tiles, rows and columns ending inside one
     (768, 530, 65),      # 32 x 64 tiles
 ])
