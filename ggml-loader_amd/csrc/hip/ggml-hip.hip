@@ -1231,10 +1231,10 @@ private:
         const int64_t cols = mm->src[1]->ne[1];
         return cols >= GEMM_MIN_COLS || (cols >= GEMM_WIDE_MIN_COLS && mm->src[0]->ne[1] >= GEMM_WIDE_MIN_ROWS);
     }
-    // narrower Q4_0 / Q8_0 products with enough 16 x 16 tiles (GEMM_MIN_TILES)
+    // narrower Q4_0 / Q8_0 products with enough 16 x 16 tiles (GEMM_MAX_MM_Q_TILES)
     static bool gemm_tiles(const ggml_tensor * mm) {
         const int64_t cols = mm->src[1]->ne[1], rows = mm->src[0]->ne[1];
-        return cols > 16 && (rows + 15) / 16 * ((cols + 15) / 16) >= GEMM_MIN_TILES;
+        return cols > 16 && (rows + 15) / 16 * ((cols + 15) / 16) > GEMM_MAX_MM_Q_TILES;
     }
     // a Q4_0 / Q8_0 mul_mat over a prefill-width batch: the int8-MFMA GEMM (same floats as the GEMV)
     bool gemm_route(const ggml_tensor * mm) const {

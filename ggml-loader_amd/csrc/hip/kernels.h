@@ -136,16 +136,22 @@ struct gemv_mat {
 // ---------------------------------------------------------------------------------------------
 // prefill GEMM on the matrix cores: y[c][r] = W[r] . x[c] (+ add[c][r]) for Q4_0 / Q8_0 weights
 // in the plane layout with Q8_0-quantized activation columns; the same floats as the GEMV.
-constexpr int GEMM_MIN_COLS = 64;   // narrower products stay on the GEMV, except:
-// an output projection this tall (an LM head) takes the GEMM from GEMM_WIDE_MIN_COLS columns: its
-// weights stream once at the GEMM's rate, where the multi-column GEMV would stage every column's
-// activation once per 16-row workgroup
+constexpr int GEMM_MIN_COLS = 64;   // narrower products stay on k_mm_q.hip or the GEMVs, except:
+// an output projection this tall (an LM head) takes the GEMM from GEMM_WIDE_MIN_COLS columns. These two lines
+// were drawn against a GEMV that staged every column once per 16 rows. Against k_mm_q.hip (us with the
+// quantization launch, k_mm_q.hip / GEMM, Q4_0, rows x 3072) the GEMM is the faster one from more than one tile
+// of 16 columns over many rows, 65536 by 16 columns 62 / 108, by 24 119 / 109, 128256 by 16 119 / 200, by 40
+// 322 / 203, and at 64 columns from many rows, 1024 10.7 / 21.5, 3072 15.7 / 21.5, 3072 by 128 27.9 / 22.2.
 constexpr int GEMM_WIDE_MIN_COLS = 16;
 constexpr int64_t GEMM_WIDE_MIN_ROWS = 65536;
-// and more than one 16-column tile takes it from this many 16 x 16 tiles (us, Q4_0, k_mm_q.hip / GEMM): 3072 x
-// 8192 by 32 columns (1024 tiles) 21.0 / 22.9, by 48 (1536) 29.1 / 23.2; 3072 x 12288 by 17 (1536) 28.9 / 25.9;
-// 3072 x 32064 by 12 (one tile of columns) 32.1 / 37.1, by 17 63.9 / 37.4; 4096 x 4096 by 63 (1024) 24.5 / 28.6
-constexpr int64_t GEMM_MIN_TILES = 1536;
+// and more than one 16-column tile takes it past this many 16 x 16 tiles, five one-wave workgroups of k_mm_q.hip
+// per CU: with more, that kernel's time goes up by a round. us, k_mm_q.hip / GEMM, by 32 columns: Q4_0 9216 x 8192
+// (1152 tiles) 55.2 / 57.9, 10240 (1280) 55.4 / 57.9, 10368 (1296) 60.3 / 57.9, 11520 (1440) 60.7 / 58.2; 10240 x 3072
+// 24.4 / 24.6, 10496 (1312) 26.6 / 24.6; Q8_0 10240 x 8192 62.8 / 56.8, 10368 68.9 / 56.9. Below the line products of
+// three and four column tiles would gain down to about 1056 tiles (6144 x 3072 by 48, 1152, 25.0 / 21.5); at 1024 none
+// does (8192 x 3072 by 32 18.9 / 21.5, 4096 x 4096 by 63 23.3 / 27.2). One column tile stays on k_mm_q.hip: 32064 x
+// 3072 by 12 (2004) 32.1 / 37.1.
+constexpr int64_t GEMM_MAX_MM_Q_TILES = 5 * 256;
 
 struct gemm_launch {
     int             type;      // GGML_TYPE_Q4_0 / Q8_0

@@ -44,8 +44,10 @@ def same(hip, cpu, build):
     (13824, 64, 4),      # a row too long for the vector kernel's LDS
     (256, 8192, 16),     # 512 tiles: K split over the waves
     (256, 8200, 16),     # 513: one wave per tile
-    (384, 12272, 32),    # 1534 tiles
-    (384, 12288, 32),    # 1536: the GEMM
+    (384, 10240, 32),    # 1280 tiles
+    (384, 10256, 32),    # 1282: the GEMM
+    (384, 12272, 32),
+    (384, 12288, 32),
     (160, 70, 9),        # not whole groups of four blocks
 ])
 def test_few_columns(hip, cpu, qtype, K, N, ncols):
