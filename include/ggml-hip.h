@@ -24,7 +24,9 @@ GGML_API ggml_backend_buffer_type_t ggml_backend_hip_buffer_type(int device);
 
 // ---- extensions of this backend (no counterpart in the reference) ----
 
-// Bytes of device scratch ggml_backend_hip_graph_compute_static can give a graph's kernels.
+// Bytes of device scratch ggml_backend_hip_graph_compute_static can give a graph's kernels: twice 64 MiB,
+// because the matrix kernels of several K-quant columns read an activation in a form of 2.25 bytes a value
+// where the one-column kernels' has 1.14, and 8 MiB for that form's whole groups of 16 columns.
 #define GGML_HIP_STATIC_SCRATCH_BYTES (136 << 20)
 
 // ggml_backend_graph_compute without any device allocation: no counterpart in the reference; for

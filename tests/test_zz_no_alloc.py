@@ -133,6 +133,29 @@ def test_static_compute_of_query_batches(hip):
         assert np.array_equal(a, b)
 
 
+def test_static_compute_of_a_large_kquant_batch(hip):
+    # 64 MiB less 0.3 of quantized values as a one-column kernel reads them: 126 MiB in the matrix kernel's form
+    K, T, N = 4096, 14300, 64
+    r = rng(9)
+    rows = r.standard_normal((50, K)).astype(np.float32)
+    pick = r.integers(0, 50, T).astype(np.int32)
+    w = quantize((r.standard_normal((N, K)) * 0.02).astype(np.float32), gl.Q4_K, impl="product")
+    core, outs = gl.libs()["core"], []
+    for fn in (core.ggml_backend_graph_compute, gl.libs()["hip"].ggml_backend_hip_graph_compute_static):
+        with Graph() as g:
+            x = g.get_rows(g.tensor(gl.F32, K, 50, data=rows), g.tensor(gl.I32, T, data=pick))
+            y = g.mul_mat(g.tensor(gl.Q4_K, K, N, data=w), x)
+            gf = core.ggml_new_graph(g.ctx)
+            core.ggml_set_output(y)
+            core.ggml_build_forward_expand(gf, y)
+            g.buf = core.ggml_backend_alloc_ctx_tensors(g.ctx, hip)
+            for t, a in g.inputs:
+                core.ggml_backend_tensor_set(t, a.ctypes.data, 0, a.nbytes)
+            assert fn(hip, gf) == 0
+            outs.append(g.read(y))
+    assert np.array_equal(*outs)
+
+
 def test_static_compute_rejects_oversized_scratch(hip):
     # 64 queries x 32 heads x 8192 positions: 64 MiB of f32 scores and 128 MiB of partial outputs in double
     big = layer_inputs(8192, 64, hd=128, n_head=32, n_head_kv=8, seed=3)
