@@ -1279,10 +1279,12 @@ void launch_attn_decode(const attn_launch & A_in, hipStream_t st) {
 //           partial sums are added in LDS (double sums, exact in practice).
 // A lane keeps its scores (4 per tile) in registers, PT tiles at most, or (PT = 0) in its own 16 bytes
 // per tile of a scratch buffer that only it reads again: no LDS in the loops, no barrier but between
-// the phases. The f64 pipe bounds it: the f64 matrix instructions (2 n_q n_kv hd multiply-adds per head,
-// 29 ns per 16x16x4 and SIMD, 72 TFLOP/s) and the vector instructions of every wave of a SIMD take turns
-// (measured: 8 vector instructions between two of them add their whole 16 ns), so what counts beside them
-// is the number of vector instructions: K and V converted F16 -> F32 -> F64, the exps in double. Two row
+// the phases. The f64 pipe bounds it: the f64 matrix instructions (2 n_q n_kv hd multiply-adds per head, 28 ns
+// per 16x16x4 and SIMD, 75 TFLOP/s) and the vector instructions of every wave of a SIMD take turns (measured,
+// profiles/rates_f64_matrix_copy_product.md: 8 vector instructions after each take 13 to 14 ns alone and add 22 to
+// 28 ns), so what counts beside them is the number of vector instructions: K and V converted F16 -> F32 -> F64, the
+// exps in double. Counted over 1000 queries and 4001 positions (profiles/activity_multi_column.md): matrix
+// instructions 52% of the SIMDs' time, vector ones 21% at 4 cycles each, conversions to double more. Two row
 // tiles per workgroup (K and V converted once for both) gained 3% at 1000 queries over 4001 positions
 // and lost 9 to 20% where the doubled workgroups fill the CUs badly (300 over 1800, 640 over 8832).
 // Measured (us a launch; before: score rows in LDS up to 2176 positions at head dim 128, K and V through

@@ -1,5 +1,7 @@
-// k_mm_q.hip — Q4_0 / Q8_0 weights times 4 to 63 activation columns on the matrix cores: multi-token
-// decode steps, prompts too short for the GEMM, and the columns of a mul_mat_id grouped by expert.
+// k_mm_q.hip — Q4_0 / Q8_0 weights times a few activation columns on the matrix cores: multi-token
+// decode steps, prompts too short for the GEMM, and the columns of a mul_mat_id grouped by expert. Mostly 4
+// to 63 columns (MM_Q_MIN_COLS, GEMM_MIN_COLS); 2 and 3 where the rows are too long for the vector kernel's
+// LDS, 64 and more where the GEMM's outputs are not 16-byte aligned.
 //
 // Per (row, column) the arithmetic is the GEMV's: exact integer block dots, the terms (sumi * d_w) * d_x
 // (Q4_0) and sumi * (d_w * d_x) (Q8_0), added in block order, so the result is the CPU reference's float.

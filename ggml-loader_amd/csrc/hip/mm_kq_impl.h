@@ -11,8 +11,8 @@
 //
 // A wave takes 16 weight rows and NT tiles of 16 columns over the whole of K, so
 // the nine running sums of its outputs stay in registers and are added in ggml's order. One
-// v_mfma_f32_16x16x32_f16 per slice l gives aux32[l] of a tile: the activations come as records
-// (q8k_act::rec) whose slices are f16 runs in MFMA operand order, and each lane decodes its own
+// v_mfma_f32_16x16x32_f16 per slice l gives aux32[l] of a tile: the activations come in a form
+// (q8k_act::x16) whose slices are f16 runs in MFMA operand order, and each lane decodes its own
 // share of a weight row (row lane % 16, the elements 64 q .. 64 q + 63 of the super-block with
 // q = lane / 16, which are k = 8q .. 8q + 7 of every slice) in registers: no weight goes through
 // LDS and a decoded operand serves all NT tiles. sc * q is exact in f16 for Q4_K (at most 945) and
@@ -27,8 +27,11 @@
 // (mm_kq_split_kernel).
 //
 // What bounds it: the VALU (per 16 x 16 tile and super-block 80 operations for the nine sums, and
-// about 120 to decode the weights, shared by the NT tiles), at 45-70% of its issue rate, the rest
-// waits at the barriers and, for small grids, CUs with two workgroups beside CUs with one. Measured
+// about 120 to decode the weights, shared by the NT tiles) together with the matrix cores. Counted
+// (profiles/activity_multi_column.md), 512 columns of Q4_K: the vector instructions fill 60% of the SIMDs'
+// time in 64 x 64 tiles and 51% in 64 x 48 ones, the matrix instructions 16% and 14%; the rest waits at the
+// barriers and, for small grids, on CUs with two workgroups beside CUs with one. Routed 64 x 32 tiles stand at
+// 34-38%, workgroups with resident columns at 62%. Measured
 // (us, with the activation's quantization) against the kernels it replaced: a prompt's gate and up
 // projections (Q4_K, K = 2560, 2 x 9728 rows, 512 columns) 200 -> 152, its down projection (K =
 // 9728, 2560 rows) 100 -> 94; 16 columns 120 -> 17.7 (K = 9728, 2560 rows), 63 columns of Q6_K 510 ->
