@@ -1280,16 +1280,16 @@ void launch_attn_decode(const attn_launch & A_in, hipStream_t st) {
 // A lane keeps its scores (4 per tile) in registers, PT tiles at most, or (PT = 0) in its own 16 bytes
 // per tile of a scratch buffer that only it reads again: no LDS in the loops, no barrier but between
 // the phases. The f64 pipe bounds it: the f64 matrix instructions (2 n_q n_kv hd multiply-adds per head, 28 ns
-// per 16x16x4 and SIMD, 75 TFLOP/s) and the vector instructions of every wave of a SIMD take turns (measured,
-// profiles/rates_f64_matrix_copy_product.md: 8 vector instructions after each take 13 to 14 ns alone and add 22 to
-// 28 ns), so what counts beside them is the number of vector instructions: K and V converted F16 -> F32 -> F64, the
-// exps in double. Counted over 1000 queries and 4001 positions (profiles/activity_multi_column.md): matrix
-// instructions 52% of the SIMDs' time, vector ones 21% at 4 cycles each, conversions to double more. Two row
+// per 16x16x4 and SIMD, 75 TFLOP/s) and the vector instructions of every wave of a SIMD take turns (measured: 8
+// vector instructions after each take 13 to 14 ns alone and add 22 to 28 ns), so what counts beside them is the
+// number of vector instructions: K and V converted F16 -> F32 -> F64, the exps in double. Counted over 1000
+// queries and 4001 positions: matrix instructions 52% of the SIMDs' time, vector ones 21% at 4 cycles each,
+// conversions to double more. Two row
 // tiles per workgroup (K and V converted once for both) gained 3% at 1000 queries over 4001 positions
 // and lost 9 to 20% where the doubled workgroups fill the CUs badly (300 over 1800, 640 over 8832).
 // Measured (us a launch; before: score rows in LDS up to 2176 positions at head dim 128, K and V through
 // LDS; past it the multi-query kernels above in groups of 64 queries): Phi-3 heads (32 x 96), 512 queries over
-// 512 positions 81 -> 66; GQA (32 heads, 8 KV, 128), 1000 over 4001 2240 -> 1480 (39 TFLOP/s).
+// 512 positions 81 -> 66; GQA (32 heads, 8 KV, 128), 1000 over 4001 2240 -> 1409 (41 TFLOP/s).
 // (f64 MFMA lane layout as above.)
 constexpr int APF_ROWS = 16;           // (query, head) rows per workgroup
 constexpr int APF_MAX_TILES = 4096;    // positions <= 65536

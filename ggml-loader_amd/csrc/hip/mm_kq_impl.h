@@ -27,12 +27,12 @@
 // (mm_kq_split_kernel).
 //
 // What bounds it: the VALU (per 16 x 16 tile and super-block 80 operations for the nine sums, and
-// about 120 to decode the weights, shared by the NT tiles) together with the matrix cores. Counted
-// (profiles/activity_multi_column.md), 512 columns of Q4_K: the vector instructions fill 60% of the SIMDs'
-// time in 64 x 64 tiles and 51% in 64 x 48 ones, the matrix instructions 16% and 14%; the rest waits at the
-// barriers and, for small grids, on CUs with two workgroups beside CUs with one. Routed 64 x 32 tiles stand at
-// 34-38%, workgroups with resident columns at 62%. Measured
-// (us, with the activation's quantization) against the kernels it replaced: a prompt's gate and up
+// about 120 to decode the weights, shared by the NT tiles) together with the matrix cores. Counted over 512
+// columns of Q4_K: the vector instructions fill 60% of the SIMDs' time in 64 x 64 tiles and 51% in 64 x 48
+// ones, the matrix instructions 16% and 14%; the rest waits at the barriers and, for small grids, on CUs
+// with two workgroups beside CUs with one. Routed 64 x 32 tiles stand at 34-38%, workgroups with
+// resident columns at 62%. Measured (us, with the activation's quantization) against the kernels it
+// replaced: a prompt's gate and up
 // projections (Q4_K, K = 2560, 2 x 9728 rows, 512 columns) 200 -> 152, its down projection (K =
 // 9728, 2560 rows) 100 -> 94; 16 columns 120 -> 17.7 (K = 9728, 2560 rows), 63 columns of Q6_K 510 ->
 // 50; the routed experts of a 384-token prompt (128 experts of 768, top 8) 3138 -> 260, of a 16-token
