@@ -2059,7 +2059,8 @@ private:
             A.out = A0.out + (int64_t) q0 * A0.out_nb1;
             const int64_t K = (int64_t) A0.n_head * A0.hd;
             if (A0.out_q.qs) A.out_q = q8_act{ A0.out_q.qs + q0 * K, A0.out_q.d + q0 * (K / 32), A0.out_q.s + q0 * (K / 32) };
-            if (A0.out_q8k.set()) A.out_q8k.x16 = A0.out_q8k.x16 + (q0 / 16) * (K / 256) * X16_BYTES;
+            if (A0.out_q8k.x16) A.out_q8k.x16 = A0.out_q8k.x16 + (q0 / 16) * (K / 256) * X16_BYTES;
+            else if (A0.out_q8k.qs) A.out_q8k = q8k_act{ A0.out_q8k.qs + q0 * K, A0.out_q8k.d + q0 * (K / 256), A0.out_q8k.bsums + q0 * (K / 16), nullptr };
             launch_attn_decode(A, st_);
         }
     }

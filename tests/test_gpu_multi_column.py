@@ -6,7 +6,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from gl import Graph, cpu_backend, gl, moe_ffn_graph, quantize, rel_err, run_on
+from gl import Graph, attention_graph, cpu_backend, gl, moe_ffn_graph, quantize, rel_err, run_on
 from test_gpu_ops import profiled
 
 pytestmark = pytest.mark.gpu
@@ -123,32 +123,47 @@ def test_kquant_many_experts(hip, cpu, qtype):
         assert np.array_equal(a, b), rel_err(a, b)
 
 
-@pytest.mark.parametrize("qtype", [gl.Q4_K, gl.Q5_K])
-@pytest.mark.parametrize("ncols", [5, 70])
-def test_kquant_weights_at_8_bytes(hip, cpu, qtype, ncols):
-    """Weights that a caller placed 8 bytes past the buffer's alignment."""
+def run_with_weights_at_8_bytes(backend, qtype, K, N, w, build):
+    """build(g, wt) with the weights 8 bytes past the alignment of a buffer of their own."""
     core = gl.libs()["core"]
-    K, N = 512, 100
-    w = qweight(qtype, K, N, 51)
-    x = rng(52).standard_normal((ncols, K)).astype(np.float32)
-
-    def run(backend):
-        buft = C.c_void_p(core.ggml_backend_get_default_buffer_type(backend))
-        buf = C.c_void_p(core.ggml_backend_buft_alloc_buffer(buft, w.nbytes + 1024))
-        with Graph() as g:
-            wt = g.tensor(qtype, K, N, data=w)
-            core.ggml_backend_tensor_alloc(buf, wt, C.c_void_p(core.ggml_backend_buffer_get_base(buf) + 8))
-            out = g.compute(backend, g.mul_mat(wt, g.tensor(gl.F32, K, ncols, data=x)))
-        core.ggml_backend_buffer_free(buf)
-        return out
-
     for name in ("ggml_backend_get_default_buffer_type", "ggml_backend_buft_alloc_buffer", "ggml_backend_buffer_get_base"):
         getattr(core, name).restype = C.c_void_p
     core.ggml_backend_get_default_buffer_type.argtypes = [C.c_void_p]
     core.ggml_backend_buft_alloc_buffer.argtypes = [C.c_void_p, C.c_size_t]
     core.ggml_backend_buffer_get_base.argtypes = [C.c_void_p]
     core.ggml_backend_tensor_alloc.argtypes = [C.c_void_p, gl.T, C.c_void_p]
-    a, b = run(hip), run(cpu)
+    buf = C.c_void_p(core.ggml_backend_buft_alloc_buffer(core.ggml_backend_get_default_buffer_type(backend), w.nbytes + 1024))
+    with Graph() as g:
+        wt = g.tensor(qtype, K, N, data=w)
+        core.ggml_backend_tensor_alloc(buf, wt, core.ggml_backend_buffer_get_base(buf) + 8)
+        out = g.compute(backend, build(g, wt))
+    core.ggml_backend_buffer_free(buf)
+    return out
+
+
+@pytest.mark.parametrize("qtype", [gl.Q4_K, gl.Q5_K])
+@pytest.mark.parametrize("ncols", [5, 70])
+def test_kquant_weights_at_8_bytes(hip, cpu, qtype, ncols):
+    """Weights that a caller placed 8 bytes past the buffer's alignment."""
+    K, N = 512, 100
+    w = qweight(qtype, K, N, 51)
+    x = rng(52).standard_normal((ncols, K)).astype(np.float32)
+    a, b = (run_with_weights_at_8_bytes(v, qtype, K, N, w, lambda g, wt: g.mul_mat(wt, g.tensor(gl.F32, K, ncols, data=x)))
+            for v in (hip, cpu))
+    assert np.array_equal(a, b), rel_err(a, b)
+
+
+def test_attention_before_weights_at_8_bytes(hip, cpu):
+    """The same of an O projection: the attention of 70 queries, in groups of 64, writes the one-column form."""
+    hd, n_head, n_head_kv, n_kv, n_new = 128, 24, 8, 2300, 70
+    r = rng(53)
+    kc, vc = (r.standard_normal((n_kv, n_head_kv, hd)).astype(np.float16) for _ in range(2))
+    q = r.standard_normal((n_new, n_head, hd)).astype(np.float32)
+    mask = np.triu(np.full((n_new, n_kv), -np.inf, dtype=np.float32), n_kv - n_new + 1)
+    K, N = n_head * hd, 64
+    w = qweight(gl.Q4_K, K, N, 54)
+    a, b = (run_with_weights_at_8_bytes(v, gl.Q4_K, K, N, w, lambda g, wt: g.mul_mat(
+        wt, attention_graph(g, hd, n_head, n_head_kv, n_kv, n_new, n_kv, kc, vc, q, mask))) for v in (hip, cpu))
     assert np.array_equal(a, b), rel_err(a, b)
 
 
