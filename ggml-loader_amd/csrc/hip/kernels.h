@@ -144,14 +144,15 @@ constexpr int GEMM_MIN_COLS = 64;   // narrower products stay on k_mm_q.hip or t
 // 322 / 203, and at 64 columns from many rows, 1024 10.7 / 21.5, 3072 15.7 / 21.5, 3072 by 128 27.9 / 22.2.
 constexpr int GEMM_WIDE_MIN_COLS = 16;
 constexpr int64_t GEMM_WIDE_MIN_ROWS = 65536;
-// and more than one 16-column tile takes it past this many 16 x 16 tiles, five one-wave workgroups of k_mm_q.hip
-// per CU: with more, that kernel's time goes up by a round. us, k_mm_q.hip / GEMM, by 32 columns: Q4_0 9216 x 8192
-// (1152 tiles) 55.2 / 57.9, 10240 (1280) 55.4 / 57.9, 10368 (1296) 60.3 / 57.9, 11520 (1440) 60.7 / 58.2; 10240 x 3072
-// 24.4 / 24.6, 10496 (1312) 26.6 / 24.6; Q8_0 10240 x 8192 62.8 / 56.8, 10368 68.9 / 56.9. Below the line products of
-// three and four column tiles would gain down to about 1056 tiles (6144 x 3072 by 48, 1152, 25.0 / 21.5); at 1024 none
-// does (8192 x 3072 by 32 18.9 / 21.5, 4096 x 4096 by 63 23.3 / 27.2). One column tile stays on k_mm_q.hip: 32064 x
-// 3072 by 12 (2004) 32.1 / 37.1.
-constexpr int64_t GEMM_MAX_MM_Q_TILES = 5 * 256;
+// and more than one 16-column tile takes it past this many 16 x 16 tiles. us, k_mm_q.hip / GEMM: one product by 32
+// columns goes up by a round past five one-wave workgroups per CU, Q4_0 10240 x 8192 (1280 tiles) 55.4 / 57.9, 10368 (1296)
+// 60.3 / 57.9, 10496 x 3072 (1312) 26.6 / 24.6, Q8_0 10240 x 8192 62.8 / 56.8. A gate / up pair, which k_mm_q.hip runs as
+// one launch with its SwiGLU, breaks even a little later; the block, Q4_0 7168 x 4096 by 35 (1344) 79.6 / 80.3, 7424 x 3072 by 48
+// (1392) 76.3 / 70.0, 5632 x 3072 by 60 (1408) 74.4 / 66.0, 12288 x 3072 by 20 (1536) 87.6 / 85.0; Q8_0 1344 94.1 / 84.7. Below the line
+// three and four column tiles would gain down to about 1056 (6144 x 3072 by 48, 1152, 25.0 / 21.5) and two lose; at 1024 all
+// do (8192 x 3072 by 32 18.9 / 21.5, 4096 x 4096 by 63 23.3 / 27.2). One column tile stays on k_mm_q.hip: 32064 x 3072 by
+// 12 (2004) 32.1 / 37.1.
+constexpr int64_t GEMM_MAX_MM_Q_TILES = 1344;
 
 struct gemm_launch {
     int             type;      // GGML_TYPE_Q4_0 / Q8_0

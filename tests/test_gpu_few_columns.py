@@ -44,8 +44,8 @@ def same(hip, cpu, build):
     (13824, 64, 4),      # a row too long for the vector kernel's LDS
     (256, 8192, 16),     # 512 tiles: K split over the waves
     (256, 8200, 16),     # 513: one wave per tile
-    (384, 10240, 32),    # 1280 tiles
-    (384, 10256, 32),    # 1282: the GEMM
+    (384, 10752, 32),    # 1344 tiles
+    (384, 10768, 32),    # 1346: the GEMM
     (384, 12272, 32),
     (384, 12288, 32),
     (160, 70, 9),        # not whole groups of four blocks
