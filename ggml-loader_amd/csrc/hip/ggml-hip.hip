@@ -2043,10 +2043,10 @@ private:
     float * prefill_buf_ = nullptr;
     int64_t prefill_bytes_ = 0;
 
-    // More queries than the fused decode path takes, over more positions than the prefill kernel
-    // takes for so few (a multi-token step deep into the context): the decode kernels, whose workgroups
-    // take 4 queries each, over up to ATT_DECODE_MAX_Q queries per launch, each launch with its own
-    // rows of Q, mask and output (same arithmetic per query).
+    // More queries than the fused decode path takes, over more positions than the prefill kernel takes
+    // for so few (a multi-token step deep into the context): the split-KV kernels, over up to
+    // ATT_DECODE_MAX_Q queries per launch, each launch with its own rows of Q, mask and output (same
+    // arithmetic per query).
     void attn_decode_grouped(const attn_launch & A0) {
         attn_launch A = A0;
         A.scratch_bytes = attn_scratch_bytes(A0.n_kv, std::min(A0.n_q, ATT_DECODE_MAX_Q), A0.n_head, A0.hd);
